@@ -1,0 +1,84 @@
+"""k_pretok's two tile sizes: texts around the edges of the small tile (768
+bytes), at the largest request that takes it and one byte past, and runs whose
+state crosses more than 64 tiles (the wave-wide look-back takes two steps),
+against the oracle."""
+
+from __future__ import annotations
+
+import re
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from conftest import kit
+
+pytestmark = pytest.mark.gpu
+
+# one family per split ruleset (laguna: cl100k inside its newline parts)
+NAMES = ["qwen3_8b", "llama_3_1_8b", "gpt2", "deepseek_v3", "gpt_oss_120b",
+         "kimi_k3", "laguna_s_2_1"]
+
+
+def _const(name: str) -> str:
+    h = Path(__file__).resolve().parents[1] / "toktier_amd" / "csrc" / "tk_device.h"
+    return re.search(rf"constexpr \w+ {name} =\s*([^;]+);", h.read_text()).group(1)
+
+
+TILE_S = int(_const("PT_TILE_S"))
+SMALL_MAX = TILE_S * 256 * 7  # PT_SMALL_MAX
+
+_TOKS: dict = {}
+
+
+def tok(name: str):
+    if name not in _TOKS:
+        import toktier_amd
+        _TOKS[name] = toktier_amd.load(name)
+    return _TOKS[name]
+
+
+def check(name: str, text: str, what) -> None:
+    want = kit(name).expected(text)
+    assert not isinstance(want, int), (name, what)
+    got = tok(name).encode(text).array
+    assert np.array_equal(got, want), (name, what)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_small_tile_edges(name):
+    """Branch atoms of the split at every alignment near a small tile's end."""
+    import soak_docs
+    rng = np.random.default_rng(71)
+    atoms = soak_docs._atoms(name)
+    for k in range(48):
+        lead = "x" * int(rng.integers(0, 66)) + " "
+        body = "".join(atoms[int(i)] for i in rng.integers(0, len(atoms), 700))
+        at = k % 8 - 4 + TILE_S * (1 + k % 3)  # the text's last byte
+        text = (lead + body).encode()[:at].decode("utf-8", "ignore")
+        check(name, text, (k, at))
+        check(name, lead + body, k)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_runs_across_many_small_tiles(name):
+    """Runs whose start or state is over 64 small tiles back: digits, letters
+    without case, marks between punctuation, whitespace, line ends."""
+    n = 65 * TILE_S + 37
+    for run in ("1234567" * (n // 7), "中" * (n // 3), "!́" * (n // 3),
+                " " * 3000 + "\n" + "\t" * 3000, "\r\n" * 2000, "Q" * n + "é"):
+        for lead in ("", "ab ", "!"):
+            check(name, lead + run + " z1", (run[:2], lead))
+
+
+@pytest.mark.parametrize("name", NAMES)
+@pytest.mark.parametrize("past", [0, 1])
+def test_largest_small_tile_request(name, past):
+    """The last size on small tiles and the first on large ones."""
+    from toktier_amd import workloads
+    n = SMALL_MAX + past
+    text = workloads._ascii_stream(
+        np.random.default_rng(5 + past),
+        workloads._Words(np.random.default_rng(6), ["the", "Of", "inter", "x9"]), n)
+    assert len(text.encode()) == n
+    check(name, text, n)

@@ -231,8 +231,8 @@ __host__ __device__ __forceinline__ uint32_t added_slot(uint32_t key,
                                                         uint32_t size) {
   return (uint32_t)(((uint64_t)(key * 0x9E3779B1u) * size) >> 32);
 }
-// packed short-piece BPE: grid of k_bpe_pack, seven waves on every SIMD
-// (blocks of four waves, 256 CUs); the eighth wave slot is left to the
+// packed short-piece BPE: grid of k_bpe_pack, at most seven waves on every
+// SIMD (blocks of four waves, 256 CUs); the eighth wave slot is left to the
 // side streams' long-piece kernels, which run beside it
 constexpr int PACK_BLOCKS = 1792;
 // k_bpe_pack merges the queued pieces of 65..128 bytes itself when at most
@@ -247,6 +247,15 @@ static_assert(CTRL_WORDS == CTRL_PSEG + PACK_XCDS * CTRL_PSEG_STRIDE,
               "one control line per segment");
 static_assert(CTRL_ROWQ + PACK_XCDS <= CTRL_VLIST, "row counters before the window list's");
 static_assert(CTRL_VLIST < CTRL_PSEG, "the window count before the segment lines");
+// k_bpe_pack's blocks for nb bytes: a wave per work unit of a segment (one
+// partial unit per class and a full one per ~128 bytes: 64 pieces, most of 3
+// to 16 bytes, or 16 of up to 32), so each takes its unit without a trip to
+// the queue counter; small requests don't dispatch and drain the whole grid.
+// (Any multiple of PACK_XCDS is correct: the units are handed out by counters.)
+__host__ __device__ inline uint32_t pack_blocks(int64_t nb) {
+  const int64_t per_seg = 4 + nb / (4 * 128 * PACK_XCDS);
+  return (uint32_t)(per_seg < PACK_BLOCKS / PACK_XCDS ? per_seg * PACK_XCDS : PACK_BLOCKS);
+}
 // slots (lanes per piece) of the length classes, and the shortest piece of
 // each class: class c holds pieces of pack_lmin(c)..pack_slot(c) bytes
 __host__ __device__ constexpr int pack_slot(int c) {
@@ -282,22 +291,34 @@ __host__ __device__ constexpr int pack_lmin(int c) {
 
 constexpr int PRETOK_TPB = 256;
 constexpr int PT_TILE = 2816;  // bytes per k_pretok block (44 start words)
+// Small requests take smaller tiles: a block's time is a serial chain over
+// its words (a wave takes a quarter of them one after another), so a request
+// whose PT_TILE tiles do not fill the chip is cut finer and spread over more
+// CUs. Up to PT_SMALL_MAX bytes there are at most as many PT_TILE_S tiles as
+// blocks fit at once (256 CUs, 7 a CU); past that the finer tiles' halos
+// (128 of 896 staged bytes) cost more than the spread gives.
+constexpr int PT_TILE_S = 768;  // 12 start words
+constexpr int64_t PT_SMALL_MAX = (int64_t)PT_TILE_S * 256 * 7;
+__host__ __device__ inline int pretok_tile(int64_t nb) {
+  return nb <= PT_SMALL_MAX ? PT_TILE_S : PT_TILE;
+}
 // k_pretok blocks: the start words 0..nwin+1 (nwin = ceil(nb / 64))
-__host__ __device__ inline int64_t pretok_tiles(int64_t nb) {
-  return (((nb + 63) / 64 + 2) * 64 + PT_TILE - 1) / PT_TILE;
+__host__ __device__ inline int64_t pretok_tiles(int64_t nb, int tile) {
+  return (((nb + 63) / 64 + 2) * 64 + tile - 1) / tile;
 }
 // Room in the piece lists: a tile holds at most pack_local_cap(c) pieces of
 // class c (every piece of pack_lmin(c) or more bytes that starts in it), so
-// the lists take PT_LOCAL_SLOTS words per tile. Segment x's lists follow
+// the lists take pack_local_slots words per tile. Segment x's lists follow
 // those of the segments before it; its class c list starts pack_local_off(c)
 // words per tile of the segment into them.
-__host__ __device__ constexpr int pack_local_cap(int c) {
-  return PT_TILE / pack_lmin(c) + 1;
+__host__ __device__ constexpr int pack_local_cap(int c, int tile) {
+  return tile / pack_lmin(c) + 1;
 }
-__host__ __device__ constexpr int pack_local_off(int c) {
-  return c == 0 ? 0 : pack_local_off(c - 1) + pack_local_cap(c - 1);
+__host__ __device__ constexpr int pack_local_off(int c, int tile) {
+  return c == 0 ? 0 : pack_local_off(c - 1, tile) + pack_local_cap(c - 1, tile);
 }
-constexpr int PT_LOCAL_SLOTS = pack_local_off(PACK_CLASSES);
+constexpr int PT_LOCAL_SLOTS = pack_local_off(PACK_CLASSES, PT_TILE);
+constexpr int PT_LOCAL_SLOTS_S = pack_local_off(PACK_CLASSES, PT_TILE_S);
 // tiles of segment x, and of the segments before it, out of ntile
 __host__ __device__ inline uint32_t pack_seg_tiles(uint32_t ntile, int x) {
   return ntile > (uint32_t)x ? (ntile - (uint32_t)x + PACK_XCDS - 1) / PACK_XCDS : 0u;
@@ -307,11 +328,12 @@ __host__ __device__ inline uint32_t pack_seg_first(uint32_t ntile, int x) {
   for (int y = 0; y < x; ++y) n += pack_seg_tiles(ntile, y);
   return n;
 }
-// start of segment x's class c list (local_off = pack_local_off(c))
+// start of segment x's class c list (slots: a tile's words of all classes,
+// local_off = pack_local_off(c))
 __host__ __device__ inline uint32_t pack_seg_list(uint32_t ntile, int x,
+                                                  uint32_t slots,
                                                   uint32_t local_off) {
-  return pack_seg_first(ntile, x) * (uint32_t)PT_LOCAL_SLOTS +
-         pack_seg_tiles(ntile, x) * local_off;
+  return pack_seg_first(ntile, x) * slots + pack_seg_tiles(ntile, x) * local_off;
 }
 constexpr int COMPACT_TPB = 256;
 constexpr int COMPACT_PER_THREAD = 32;

@@ -218,12 +218,16 @@ __device__ __forceinline__ void push_pair(uint32_t* list, uint32_t* count,
 // packed waves by length class; longer ones take the long-piece stages.
 constexpr int PIECE_NONE = -1, PIECE_ONE = -2, PIECE_TWO = -3, PIECE_LONG = -4;
 
-__constant__ uint32_t PACK_LOCAL_OFF[PACK_CLASSES] = {
-    pack_local_off(0), pack_local_off(1), pack_local_off(2),
-    pack_local_off(3), pack_local_off(4), pack_local_off(5),
-    pack_local_off(6), pack_local_off(7), pack_local_off(8),
-    pack_local_off(9), pack_local_off(10), pack_local_off(11),
-    pack_local_off(12)};
+// (row 0: PT_TILE tiles, row 1: PT_TILE_S)
+#define TK_LOCAL_OFFS(T)                                              \
+  {pack_local_off(0, T), pack_local_off(1, T), pack_local_off(2, T),   \
+   pack_local_off(3, T), pack_local_off(4, T), pack_local_off(5, T),   \
+   pack_local_off(6, T), pack_local_off(7, T), pack_local_off(8, T),   \
+   pack_local_off(9, T), pack_local_off(10, T), pack_local_off(11, T), \
+   pack_local_off(12, T)}
+__constant__ uint32_t PACK_LOCAL_OFF[2][PACK_CLASSES] = {
+    TK_LOCAL_OFFS(PT_TILE), TK_LOCAL_OFFS(PT_TILE_S)};
+#undef TK_LOCAL_OFFS
 static_assert(PACK_CLASSES == 13, "PACK_LOCAL_OFF lists every class");
 
 __device__ __forceinline__ int pack_class(int L) {  // 2 <= L <= 64
@@ -384,28 +388,31 @@ __device__ __forceinline__ uint64_t nrun_load(const uint64_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 constexpr int PT_HALO = 64;
-constexpr int PT_SPAN = PT_TILE + 2 * PT_HALO;
 constexpr int PT_PAD = 80;  // >= PT_HALO + 4, a multiple of 16
-constexpr int PT_BYTES = PT_TILE + 2 * PT_PAD;
-constexpr int PT_DMW = PT_TILE / 64 + 6;  // doc-mask words from tile word - 3
+// the staged sizes of a tile of TILE bytes: entries, bytes, and doc-mask
+// words from tile word - 3
+constexpr int pt_span(int tile) { return tile + 2 * PT_HALO; }
+constexpr int pt_bytes(int tile) { return tile + 2 * PT_PAD; }
+constexpr int pt_dmw(int tile) { return tile / 64 + 6; }
 
 // LCtx answers from a block's LDS tile and falls back to GCtx for
 // positions outside it (long digit / whitespace runs, rare).
+template <int TILE>
 struct LCtx {
   GCtx g;
-  const uint32_t* se;  // entries of positions [lo, lo + PT_SPAN)
+  const uint32_t* se;  // entries of positions [lo, lo + pt_span)
   int64_t lo;
-  const uint64_t* sdm;  // doc-mask words [wlo, wlo + PT_DMW)
+  const uint64_t* sdm;  // doc-mask words [wlo, wlo + pt_dmw)
   int64_t wlo;
 
   __device__ __forceinline__ bool in(int64_t p) const {
-    return (uint64_t)(p - lo) < (uint64_t)PT_SPAN;
+    return (uint64_t)(p - lo) < (uint64_t)pt_span(TILE);
   }
   __device__ __forceinline__ bool ds(int64_t i) const {
     if (i == 0) return true;
     if (!g.dm) return false;
     const int64_t k = (i >> 6) - wlo;
-    if ((uint64_t)k < (uint64_t)PT_DMW) return (sdm[k] >> (i & 63)) & 1;
+    if ((uint64_t)k < (uint64_t)pt_dmw(TILE)) return (sdm[k] >> (i & 63)) & 1;
     return g.ds(i);
   }
   __device__ __forceinline__ Ch at(int64_t p) const {
@@ -1218,23 +1225,29 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* total)
 
 // ------------------------------------------------------ 1. pretokenize
 
-// One block per PT_TILE bytes (PT_TILE / 64 start words). Stage the bytes, decode
+// One block per TILE bytes (TILE / 64 start words). Stage the bytes, decode
 // every position of the tile and its halo into LDS entries, then each wave
 // takes one 64-byte word at a time, lane = byte, and ballots the start bits
 // into the word. Positions inside the block are 32-bit offsets from lo (the
 // first entry); RS is the ruleset, DM whether document starts are marked.
-template <int RS, bool DM>
+// TILE (pretok_tile): a block's words run one after another in four waves, so
+// a request of a few PT_TILE tiles takes one block's time on a chip that is
+// mostly idle; PT_TILE_S tiles cut that chain to three words a wave. Own
+// duration, large against small tiles: 65,536 chars 34 -> 15 us, 1,000,003
+// chars of chat 56 -> 31 us; 4,194,304 chars keep the large tile (73 us).
+template <int RS, bool DM, int TILE>
 __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7))) void k_pretok(DevTables t, DevWork w,
                                                        int64_t nwords) {
-  __shared__ __align__(16) uint8_t sb[PT_BYTES];
-  __shared__ uint32_t se[PT_SPAN];
+  constexpr int SPAN = pt_span(TILE), BYTES = pt_bytes(TILE), DMW = pt_dmw(TILE);
+  __shared__ __align__(16) uint8_t sb[BYTES];
+  __shared__ uint32_t se[SPAN];
   // the NFC quick-check value of each span position's code point
-  __shared__ uint8_t snfc[PT_SPAN];
-  __shared__ uint64_t sdm[PT_DMW];
-  __shared__ uint64_t sw[PT_TILE / 64 + 1];  // the tile's start words + next
+  __shared__ uint8_t snfc[SPAN];
+  __shared__ uint64_t sdm[DMW];
+  __shared__ uint64_t sw[TILE / 64 + 1];  // the tile's start words + next
   __shared__ uint32_t lcnt[PACK_CLASSES];
-  // pieces over 64 bytes that start in the tile (at most PT_TILE / 65)
-  __shared__ uint32_t llong[PT_TILE / 64], nlong, longbase;
+  // pieces over 64 bytes that start in the tile (at most TILE / 65)
+  __shared__ uint32_t llong[TILE / 64], nlong, longbase;
   // the first 256 code points' class and NFC value and the 256 byte ids,
   // one 32-bit word per entry (LTAB_*): LDS copies for the common case (one
   // entry per thread; 32-bit words, so the compiler keeps the LDS and HBM
@@ -1247,8 +1260,8 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   // first word after the tile: N-class character starts, run breaks (other
   // character starts and document starts), and the N characters of the run
   // at the word's end
-  __shared__ uint64_t gNL[PT_TILE / 64 + 2], gBR[PT_TILE / 64 + 2];
-  __shared__ uint32_t gC[PT_TILE / 64 + 1];
+  __shared__ uint64_t gNL[TILE / 64 + 2], gBR[TILE / 64 + 2];
+  __shared__ uint32_t gC[TILE / 64 + 1];
   // (o200k) the functions of the words before the waves' blocks, the
   // blocks' functions, and the blocks' entry states
   __shared__ uint32_t o2w[4][4], o2b[4][4];
@@ -1262,10 +1275,10 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
                 ((uint32_t)t.cls[tid] << LTAB_CLS) |
                 ((w.check_nfc ? (uint32_t)t.nfc[tid] : 0u) << LTAB_NFC);
   }
-  const int64_t base = (int64_t)blockIdx.x * PT_TILE;
+  const int64_t base = (int64_t)blockIdx.x * TILE;
   const int64_t nb = w.nb;
   const bool al = ((uintptr_t)w.text & 15) == 0;
-  for (int j = tid; j < PT_BYTES / 16; j += PRETOK_TPB) {
+  for (int j = tid; j < BYTES / 16; j += PRETOK_TPB) {
     const int64_t p = base - PT_PAD + 16 * j;
     uint4 v;
     if (al && p >= 0 && p + 16 <= nb) {
@@ -1286,7 +1299,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   // (block 0) the control slot of the next call; the last block takes the
   // tails.
   {
-    constexpr int64_t TW = PT_TILE / 64;
+    constexpr int64_t TW = TILE / 64;
     const int64_t wd0 = (base >> 6);
     const int64_t dw0 = (wd0 + 63) / 64, dw1 = (wd0 + TW + 63) / 64;
     const bool last = blockIdx.x == gridDim.x - 1;
@@ -1310,7 +1323,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   if (DM) {
     const int64_t nmw = nb / 64 + 2;  // words the caller's mask holds
     int nz = 0;
-    for (int j = tid; j < PT_DMW; j += PRETOK_TPB) {
+    for (int j = tid; j < DMW; j += PRETOK_TPB) {
       const int64_t wd = wlo + j;
       const uint64_t v = (wd >= 0 && wd < nmw) ? w.docmask[wd] : 0;
       sdm[j] = v;
@@ -1323,8 +1336,8 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   const int64_t lo = base - PT_HALO;
   // entries within the text: local offsets [jlo, jhi)
   const int jlo = lo < 0 ? (int)(-lo) : 0;
-  const int jhi = nb - lo < PT_SPAN ? (int)(nb - lo) : PT_SPAN;
-  for (int j = tid; j < PT_SPAN; j += PRETOK_TPB) {
+  const int jhi = nb - lo < SPAN ? (int)(nb - lo) : SPAN;
+  for (int j = tid; j < SPAN; j += PRETOK_TPB) {
     const int sj = j + (PT_PAD - PT_HALO);  // its byte in sb
     uint32_t e = 0;
     uint8_t snf = 0;
@@ -1400,7 +1413,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   // before a digit, and a run can be any length. Per word of the span from
   // the halo word on, the N-class character starts (gNL) and the run breaks
   // (gBR: the starts of other characters, and document starts, where a run
-  // begins), index k + 1 for word k (-1: the halo word, PT_TILE / 64: the
+  // begins), index k + 1 for word k (-1: the halo word, TILE / 64: the
   // first word after the tile, which the start words recompute); thread 0
   // counts the run's N characters at every word end up to the tile's (gC,
   // index k + 1 for tile word k, 0 for the halo word). A run that reaches
@@ -1412,7 +1425,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   uint32_t st = 0;  // status bits of the tile
   const bool groups = (RS == 0 || RS == RS_DEEPSEEK || RS == RS_O200K) && t.dmax > 1;
   if (groups) {
-    for (int k = wv - 1; k <= PT_TILE / 64; k += PRETOK_TPB / 64) {
+    for (int k = wv - 1; k <= TILE / 64; k += PRETOK_TPB / 64) {
       const int64_t p = base + 64 * k + lane;
       const int L = PT_HALO + 64 * k + lane;
       const bool ld = p >= 0 && p < nb && !is_cont(sb[L + (PT_PAD - PT_HALO)]);
@@ -1432,7 +1445,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       // run at the word's end, as a segmented prefix sum (a word with a
       // break restarts the run at its last break; a document start that is
       // an N character opens the run and counts).
-      constexpr int TW = PT_TILE / 64;
+      constexpr int TW = TILE / 64;
       static_assert(TW < 64, "a lane per tile word");
       const bool act = lane >= 1 && lane <= TW;
       const uint64_t bw = act ? gBR[lane] : 0, nw = act ? gNL[lane] : 0;
@@ -1453,39 +1466,49 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       const int fb = bm ? __builtin_ctzll(bm) - 1 : TW;
       const uint32_t run_end = (uint32_t)__builtin_amdgcn_readlane((int)run, TW);
       uint32_t c0 = 0;
-      if (lane == 0) {
-        if (w.nrun)
-          nrun_store(&w.nrun[blockIdx.x], ((uint64_t)w.seq << 32) |
-                                              (fb == TW ? NRUN_FULL : 0) | run_end);
-        if (gBR[0]) {
-          const uint64_t b0 = gBR[0], n0 = gNL[0];
-          const int h = 63 - __builtin_clzll(b0);
-          c0 = (uint32_t)__popcll(n0 & ~mask_le(h)) + (uint32_t)((n0 >> h) & 1);
-        } else if (gNL[0] && w.nrun) {
-          // the run reaches back past the halo: the tiles before it
-          WaitBound wb;
-          for (int64_t u = (int64_t)blockIdx.x - 1; u >= 0; --u) {
-            uint64_t v;
-            while ((uint32_t)((v = nrun_load(&w.nrun[u])) >> 32) != w.seq) {
-              if (wb.expired(w.wait_ticks)) break;
-              __builtin_amdgcn_s_sleep(2);
-            }
-            if ((uint32_t)(v >> 32) != w.seq) {
-              st |= ST_STALL_PRETOK;
-              break;
-            }
-            c0 += (uint32_t)(v & (NRUN_FULL - 1));
-            if (!(v & NRUN_FULL)) break;
+      if (lane == 0 && w.nrun)
+        nrun_store(&w.nrun[blockIdx.x], ((uint64_t)w.seq << 32) |
+                                            (fb == TW ? NRUN_FULL : 0) | run_end);
+      if (gBR[0]) {
+        const uint64_t b0 = gBR[0], n0 = gNL[0];
+        const int h = 63 - __builtin_clzll(b0);
+        c0 = (uint32_t)__popcll(n0 & ~mask_le(h)) + (uint32_t)((n0 >> h) & 1);
+      } else if (gNL[0] && w.nrun) {
+        // The run reaches back past the halo: the tiles before it, 64 a
+        // step (lane l the l-th tile back), up to the nearest one that the
+        // run does not span whole. (One tile a step cost a round trip
+        // each: a million-digit run spans 1,300 small tiles.)
+        WaitBound wb;
+        bool more = true;
+        for (int64_t top = (int64_t)blockIdx.x - 1; more && top >= 0; top -= 64) {
+          const int64_t u = top - lane;
+          uint64_t v = (uint64_t)w.seq << 32;  // before tile 0: an empty tile
+          uint64_t ends, wait;
+          for (;;) {
+            if (u >= 0) v = nrun_load(&w.nrun[u]);
+            const bool pub = (uint32_t)(v >> 32) == w.seq;
+            ends = __ballot(pub && !(v & NRUN_FULL));
+            const int l = ends ? __builtin_ctzll(ends) : 64;
+            wait = __ballot(!pub && lane < l);
+            if (!wait || __any(wb.expired(w.wait_ticks))) break;
+            __builtin_amdgcn_s_sleep(2);
           }
+          if (wait) {
+            st |= ST_STALL_PRETOK;
+            break;
+          }
+          const int l = ends ? __builtin_ctzll(ends) : 63;
+          const uint32_t n = lane <= l ? (uint32_t)(v & (NRUN_FULL - 1)) : 0u;
+          c0 += (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(n, lane), 63);
+          more = ends == 0;
         }
-        gC[0] = c0;
       }
-      c0 = (uint32_t)__shfl((int)c0, 0);
+      if (lane == 0) gC[0] = c0;
       if (act && lane <= fb) gC[lane] = run + c0;
     }
     __syncthreads();
   }
-  const LCtx c{GCtx{w.text, nb, DM ? w.docmask : nullptr, t.cls}, se, lo, sdm, wlo};
+  const LCtx<TILE> c{GCtx{w.text, nb, DM ? w.docmask : nullptr, t.cls}, se, lo, sdm, wlo};
   // document start at local offset L: position 0, or a marked doc head
   const int Lz = lo <= 0 ? (int)(-lo) : -1;
   auto prv = [&](int L) {  // local offset of the character before L
@@ -1499,7 +1522,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   auto start_words = [&](auto dflag) {
     constexpr bool D = decltype(dflag)::value;
     // every span position's mask word is staged (words tile - 1 .. tile +
-    // PT_TILE / 64 of the PT_DMW from tile - 3), so D reads LDS only
+    // TILE / 64 of the DMW from tile - 3), so D reads LDS only
     auto ds = [&](int L) {
       if (!D) return L == Lz;
       const int64_t i = lo + L;
@@ -1522,7 +1545,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       // (lo_st == 0: position 0 stopped the loop above; guarded all the same)
       return lo_st > 0 ? ds_stop_hbm(w.text, c.g.dm, lo_st - 1) : (int64_t)-1;
     };
-    for (int k = wv; k <= PT_TILE / 64; k += PRETOK_TPB / 64) {
+    for (int k = wv; k <= TILE / 64; k += PRETOK_TPB / 64) {
       const int64_t wd = (base >> 6) + k;
       if (wd >= nwords) {  // past the sentinel words: all starts
         if (lane == 0) sw[k] = ~0ULL;
@@ -1569,7 +1592,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       x.h3 = x.h2 && !ds(L2);
       x.h4 = x.h3 && !ds(L3);
       const int Ln = Li + 1 + (int)((e >> 25) & 3);
-      const bool nin = Ln < PT_SPAN;
+      const bool nin = Ln < SPAN;
       x.hn = lo + Ln < nb && !ds(Ln);
       x.cn = nin ? se[Ln] : 0u;
       int r = !nin ? -1
@@ -1646,7 +1669,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
             bool more = false, known = false;
             for (int L = Ln;;) {
               if (lo + L >= nb || ds(L)) { known = true; break; }
-              if (L >= PT_SPAN) break;
+              if (L >= SPAN) break;
               const uint32_t eq = se[L];
               if (!kws(kcl(eq))) { known = true; break; }
               if (crlf(ecp(eq))) { more = known = true; break; }
@@ -1704,7 +1727,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       if (DM && w.litb) m &= ~w.litb[wd];
       if (lane == 0) {
         sw[k] = m;
-        if (k < PT_TILE / 64) w.starts[wd] = m;
+        if (k < TILE / 64) w.starts[wd] = m;
       }
     }
   };
@@ -1720,18 +1743,19 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   // blocks' entries. Every tile publishes the state after it.
   auto o2k_words = [&](auto dflag) {
     constexpr bool D = decltype(dflag)::value;
+    static_assert(TILE % PRETOK_TPB == 0, "the waves take equal blocks of words");
     auto ds = [&](int L) {
       if (!D) return L == Lz;
       const int64_t i = lo + L;
       return i == 0 || ((sdm[(i >> 6) - wlo] >> (i & 63)) & 1) != 0;
     };
-    constexpr int WPB = PT_TILE / 64 / (PRETOK_TPB / 64);  // words per wave
+    constexpr int WPB = TILE / 64 / (PRETOK_TPB / 64);  // words per wave
     constexpr int NST = o2_nst<RS>();
     constexpr int W = o2_words<RS>();
     using Fn = O2Fn<W>;
     constexpr uint32_t ALL = (1u << NST) - 1;
     const bool contr = t.contractions != 0;
-    // the lane's transition and start bits in word k (-1 .. PT_TILE / 64);
+    // the lane's transition and start bits in word k (-1 .. TILE / 64);
     // positions outside the text and inside a character pass the state on
     auto lane_fn = [&](int k, bool need_g, Fn* f, uint32_t* g) {
       const int64_t i = base + 64 * k + lane;
@@ -1782,7 +1806,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
         }
       }
       const int Ln = Li + 1 + (int)((e >> 25) & 3);
-      if (Ln < PT_SPAN) {
+      if (Ln < SPAN) {
         h1 = lo + Ln < nb && !ds(Ln);
         if (h1) x1 = se[Ln];
       } else {
@@ -1851,7 +1875,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       if (DM && w.litb) m &= ~w.litb[wd];
       if (lane == 0) {
         sw[k] = m;
-        if (k < PT_TILE / 64) w.starts[wd] = m;
+        if (k < TILE / 64) w.starts[wd] = m;
       }
       return (uint32_t)__builtin_amdgcn_readlane((int)sj, 63);
     };
@@ -1877,62 +1901,77 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       carry = o2w[wv][0] & 0xFFu;
     } else {
       Fn B = o2_ident<W>();
+#pragma unroll 1  // (a small tile's three words: the code is long enough once)
       for (int k = k0; k < k0 + WPB; ++k) B = o2_then(B, word_fn(k));
       if (lane == 0)
         for (int q = 0; q < W; ++q) o2b[wv][q] = B.d[q];
       __syncthreads();
-      if (tid == 0) {
+      if (wv == 0) {
         Fn A = lds_fn(o2b, 0);
         for (int j = 1; j < PRETOK_TPB / 64; ++j) A = o2_then(A, lds_fn(o2b, j));
-        uint32_t entry = O2_FRESH;
+        uint32_t entry;
         const Fn H = lds_fn(o2w, 0);
         if (o2_const<RS>(H)) {
           entry = o2_at(H, 0);
         } else {
-          o2_publish(op, w.seq, O2_AGG, o2_pack<RS>(A), 0);
-          // G: the function of the tiles after u up to this one
+          if (lane == 0) o2_publish(op, w.seq, O2_AGG, o2_pack<RS>(A), 0);
+          // G: the function of the tiles looked at, up to this one. 64
+          // tiles a step, lane 63 the nearest (lanes in text order, so the
+          // wave's scan composes them): only the tiles after the last one
+          // whose function is constant have to be published. (One tile a
+          // step waited on its predecessor's in turn, a round trip each.)
           Fn G = o2_ident<W>();
-          bool done = false;
           WaitBound wb;
-          for (int64_t u = (int64_t)blockIdx.x - 1; u >= 0 && !done; --u) {
-            const uint64_t* q = w.ostate + 2 * u;
-            uint64_t v1;
-            while ((uint32_t)((v1 = __hip_atomic_load(q + 1, __ATOMIC_ACQUIRE,
-                                                      __HIP_MEMORY_SCOPE_AGENT)) >> 32) !=
-                   w.seq) {
-              if (wb.expired(w.wait_ticks)) break;
+          bool stall = false;
+          for (int64_t top = (int64_t)blockIdx.x - 1; !o2_const<RS>(G) && !stall;
+               top -= 64) {
+            const int64_t u = top - 63 + lane;
+            // (before tile 0 nothing came: position 0 starts a document)
+            bool pub = u < 0;
+            Fn f = u < 0 ? o2_rep<W>(O2_FRESH) : o2_ident<W>();
+            for (;;) {
+              if (!pub) {
+                const uint64_t* q = w.ostate + 2 * u;
+                const uint64_t v1 =
+                    __hip_atomic_load(q + 1, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+                pub = (uint32_t)(v1 >> 32) == w.seq;
+                if (pub && ((v1 >> 30) & 3) == O2_INCL) {
+                  f = o2_rep<W>((uint32_t)(v1 >> 26) & 15);
+                } else if (pub) {
+                  const uint64_t v0 =
+                      __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                  f = o2_unpack<RS>((uint32_t)v0 | ((v1 & 0xFFFFF) << 32));
+                }
+              }
+              const uint64_t cm = __ballot(pub && o2_const<RS>(f));
+              const int last = cm ? 63 - __builtin_clzll(cm) : -1;
+              if (!__ballot(!pub && lane > last)) break;
+              if (__any(wb.expired(w.wait_ticks))) {
+                stall = true;
+                break;
+              }
               __builtin_amdgcn_s_sleep(2);
             }
-            if ((uint32_t)(v1 >> 32) != w.seq) {
-              st |= ST_STALL_PRETOK;
-              done = true;
-            } else if (((v1 >> 30) & 3) == O2_INCL) {
-              entry = o2_at(G, (uint32_t)(v1 >> 26) & 15);
-              done = true;
-            } else {
-              const uint64_t v0 = __hip_atomic_load(q, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT);
-              G = o2_then(o2_unpack<RS>((uint32_t)v0 | ((v1 & 0xFFFFF) << 32)), G);
-              if (o2_const<RS>(G)) {
-                entry = o2_at(G, 0);
-                done = true;
-              }
-            }
+            G = o2_then(o2_lane63(o2_scan(f)), G);
           }
-          // (past tile 0 nothing came before: position 0 starts a document)
-          if (!done) entry = o2_at(G, O2_FRESH);
+          if (stall) st |= ST_STALL_PRETOK;
+          entry = o2_at(G, O2_FRESH);
         }
-        o2_publish(op, w.seq, O2_INCL, 0, o2_at(A, entry));
-        o2e[0] = entry;
-        for (int j = 1; j < PRETOK_TPB / 64; ++j) o2e[j] = o2_at(lds_fn(o2b, j - 1), o2e[j - 1]);
+        if (lane == 0) {
+          o2_publish(op, w.seq, O2_INCL, 0, o2_at(A, entry));
+          o2e[0] = entry;
+          for (int j = 1; j < PRETOK_TPB / 64; ++j)
+            o2e[j] = o2_at(lds_fn(o2b, j - 1), o2e[j - 1]);
+        }
       }
       __syncthreads();
       carry = o2e[wv];
     }
+#pragma unroll 1
     for (int k = k0; k < k0 + WPB; ++k) carry = word(k, carry);
     if (wv == PRETOK_TPB / 64 - 1) {
       if (fast && lane == 0) o2_publish(op, w.seq, O2_INCL, 0, carry);
-      word(PT_TILE / 64, carry);
+      word(TILE / 64, carry);
     }
   };
   if constexpr (RS == RS_O200K || RS == RS_KIMI) {
@@ -1951,7 +1990,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   // room in its segment's class lists, one counter update per class, and
   // writes the positions there.
   const bool two = !t.ignore_merges;
-  for (int k = wv; k < PT_TILE / 64; k += PRETOK_TPB / 64) {
+  for (int k = wv; k < TILE / 64; k += PRETOK_TPB / 64) {
     const int64_t a = base + 64 * k + lane;
     if (a >= nb) break;  // (positions only grow along the loop)
     int kind = piece_kind(sw[k], sw[k + 1], lane, two);
@@ -1982,7 +2021,8 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   // once every start word is known)
   if (tid < PACK_CLASSES && lcnt[tid]) {
     const int x = blockIdx.x % PACK_XCDS;
-    lbase[tid] = pack_seg_list(gridDim.x, x, PACK_LOCAL_OFF[tid]) +
+    constexpr uint32_t slots = TILE == PT_TILE_S ? PT_LOCAL_SLOTS_S : PT_LOCAL_SLOTS;
+    lbase[tid] = pack_seg_list(gridDim.x, x, slots, PACK_LOCAL_OFF[TILE == PT_TILE_S][tid]) +
                  atomicAdd(&w.pseg[x * CTRL_PSEG_STRIDE + CTRL_PSEG_COUNT + tid],
                            lcnt[tid]);
   } else if (tid == 64 && nlong) {
@@ -1990,7 +2030,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   }
   __syncthreads();
   {
-    const int nt = nb - base < PT_TILE ? (int)(nb - base) : PT_TILE;
+    const int nt = nb - base < TILE ? (int)(nb - base) : TILE;
     for (int i = tid; i < nt; i += PRETOK_TPB) {
       const uint32_t e = se[i];
       if (e) w.plist[lbase[(e & 15) - 1] + (e >> 4)] = (uint32_t)(base + i);
@@ -2020,26 +2060,29 @@ void launch_ev(void (*k)(KArgs...), dim3 grid, dim3 block, hipStream_t s,
     hipLaunchKernelGGL(k, grid, block, 0, s, args...);
 }
 
+template <int RS>
+void launch_pretok_rs(const DevTables& t, const DevWork& w, hipStream_t s,
+                      hipEvent_t start, hipEvent_t stop) {
+  const int64_t nwords = (w.nb + 63) / 64 + 2;  // words 0..nwin+1
+  const int tile = pretok_tile(w.nb);
+  const dim3 g((uint32_t)pretok_tiles(w.nb, tile)), b(PRETOK_TPB);
+  const bool dm = w.docmask != nullptr;
+  if (tile == PT_TILE_S)
+    launch_ev(dm ? k_pretok<RS, true, PT_TILE_S> : k_pretok<RS, false, PT_TILE_S>, g, b,
+              s, start, stop, t, w, nwords);
+  else
+    launch_ev(dm ? k_pretok<RS, true, PT_TILE> : k_pretok<RS, false, PT_TILE>, g, b, s,
+              start, stop, t, w, nwords);
+}
+
 hipError_t launch_pretok(const DevTables& t, const DevWork& w, hipStream_t s,
                          hipEvent_t start, hipEvent_t stop) {
-  const int64_t nwords = (w.nb + 63) / 64 + 2;  // words 0..nwin+1
-  const dim3 g((uint32_t)pretok_tiles(w.nb)), b(PRETOK_TPB);
-  const bool dm = w.docmask != nullptr;
-  if (t.ruleset == 1) {
-    if (dm) launch_ev(k_pretok<1, true>, g, b, s, start, stop, t, w, nwords);
-    else launch_ev(k_pretok<1, false>, g, b, s, start, stop, t, w, nwords);
-  } else if (t.ruleset == RS_DEEPSEEK) {
-    if (dm) launch_ev(k_pretok<RS_DEEPSEEK, true>, g, b, s, start, stop, t, w, nwords);
-    else launch_ev(k_pretok<RS_DEEPSEEK, false>, g, b, s, start, stop, t, w, nwords);
-  } else if (t.ruleset == RS_O200K) {
-    if (dm) launch_ev(k_pretok<RS_O200K, true>, g, b, s, start, stop, t, w, nwords);
-    else launch_ev(k_pretok<RS_O200K, false>, g, b, s, start, stop, t, w, nwords);
-  } else if (t.ruleset == RS_KIMI) {
-    if (dm) launch_ev(k_pretok<RS_KIMI, true>, g, b, s, start, stop, t, w, nwords);
-    else launch_ev(k_pretok<RS_KIMI, false>, g, b, s, start, stop, t, w, nwords);
-  } else {
-    if (dm) launch_ev(k_pretok<0, true>, g, b, s, start, stop, t, w, nwords);
-    else launch_ev(k_pretok<0, false>, g, b, s, start, stop, t, w, nwords);
+  switch (t.ruleset) {
+    case 1: launch_pretok_rs<1>(t, w, s, start, stop); break;
+    case RS_DEEPSEEK: launch_pretok_rs<RS_DEEPSEEK>(t, w, s, start, stop); break;
+    case RS_O200K: launch_pretok_rs<RS_O200K>(t, w, s, start, stop); break;
+    case RS_KIMI: launch_pretok_rs<RS_KIMI>(t, w, s, start, stop); break;
+    default: launch_pretok_rs<0>(t, w, s, start, stop);
   }
   return hipGetLastError();
 }
@@ -2661,8 +2704,11 @@ void k_bpe_pack(DevTables t, DevWork w) {
       mo[lane] = ko ? incl - lk : ~0u;
       mk[lane] = oc;
       mg2[lane] = make_uint2(cnt, geo);
-      ml[lane] = cl ? pack_seg_list((uint32_t)pretok_tiles(w.nb), x,
-                                    PACK_LOCAL_OFF[lane])
+      const int tile = pretok_tile(w.nb);
+      const bool small = tile == PT_TILE_S;
+      ml[lane] = cl ? pack_seg_list((uint32_t)pretok_tiles(w.nb, tile), x,
+                                    small ? PT_LOCAL_SLOTS_S : PT_LOCAL_SLOTS,
+                                    PACK_LOCAL_OFF[small][lane])
                     : 0u;
     }
     const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
@@ -2674,7 +2720,7 @@ void k_bpe_pack(DevTables t, DevWork w) {
     // (long_prep_step). The last of them opens the gate: how many pieces
     // are over 64 bytes and how many over WIDE_MAX, then the call's number
     // (with no long piece, wave 0 of block 0 does).
-    constexpr uint32_t GW = PACK_BLOCKS * 4;
+    const uint32_t GW = gridDim.x * 4;
     const uint32_t n = nl;
     const uint32_t P = (n + 63) / 64 < GW ? (n + 63) / 64 : GW;
     const uint32_t gw = blockIdx.x * 4 + wv;
@@ -2711,7 +2757,7 @@ void k_bpe_pack(DevTables t, DevWork w) {
   // in scalar registers)
   const uint32_t total = __builtin_amdgcn_readfirstlane(mtot);
   uint32_t* const queue = w.pseg + x * CTRL_PSEG_STRIDE;
-  constexpr uint32_t G = (PACK_BLOCKS / PACK_XCDS) * 4;  // waves per XCD
+  const uint32_t G = (gridDim.x / PACK_XCDS) * 4;  // waves per XCD
   uint32_t u0 = (blockIdx.x / PACK_XCDS) * 4 + wv;  // the first unit
   for (bool first_unit = true;; first_unit = false) {
     if (!first_unit) {
@@ -2812,7 +2858,7 @@ void k_bpe_pack(DevTables t, DevWork w) {
 
 hipError_t launch_bpe_pack(const DevTables& t, const DevWork& w, hipStream_t s,
                            hipEvent_t start, hipEvent_t stop) {
-  launch_ev(k_bpe_pack, dim3(PACK_BLOCKS), dim3(256), s, start, stop, t, w);
+  launch_ev(k_bpe_pack, dim3(pack_blocks(w.nb)), dim3(256), s, start, stop, t, w);
   return hipGetLastError();
 }
 

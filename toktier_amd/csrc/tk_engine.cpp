@@ -247,7 +247,13 @@ size_t carve(Workspace& w, uint8_t* base, size_t cap) {
   const size_t nblk = cap / tk::COMPACT_BLOCK + 2;
   const size_t long_cap = cap / 32 + 64;
   const size_t seg_cap = cap / 2 + 64;
-  const int64_t tiles = tk::pretok_tiles((int64_t)cap);
+  // the tiles and list words of the largest request of either tile size
+  const int64_t small = std::min((int64_t)cap, tk::PT_SMALL_MAX);
+  const int64_t tiles_b = tk::pretok_tiles((int64_t)cap, tk::PT_TILE);
+  const int64_t tiles_s = tk::pretok_tiles(small, tk::PT_TILE_S);
+  const int64_t tiles = std::max(tiles_b, tiles_s);
+  const int64_t list_words = std::max(tk::PT_LOCAL_SLOTS * tiles_b,
+                                      tk::PT_LOCAL_SLOTS_S * tiles_s);
   take(w.text, cap + 64);
   take(w.starts, words);
   take(w.docmask, words);
@@ -271,7 +277,7 @@ size_t carve(Workspace& w, uint8_t* base, size_t cap) {
   take(w.blkcount, nblk);
   take(w.blkprefix, nblk);
   take(w.cstat, nblk);
-  take(w.plist, (size_t)tk::PT_LOCAL_SLOTS * tiles);
+  take(w.plist, (size_t)list_words);
   take(w.lits, words);
   take(w.litb, words);
   take(w.docmask_lit, words);
@@ -472,7 +478,7 @@ tk::DevWork make_work(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   w.npass = ctrl + tk::CTRL_PASS;
   w.dirty_cur = ws.dirty_cur;
   w.dirty_next = ws.dirty_next;
-  w.plist = ws.plist;  // (tiles * PT_LOCAL_SLOTS < 2^32 for nb <= 1 GiB)
+  w.plist = ws.plist;  // (its words are below 2^32 for nb <= 1 GiB)
   w.pseg = ctrl + tk::CTRL_PSEG;
   w.nbig = ctrl + tk::CTRL_BIG;
   w.prepdone = ctrl + tk::CTRL_PREP;
