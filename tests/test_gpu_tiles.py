@@ -82,3 +82,25 @@ def test_largest_small_tile_request(name, past):
         workloads._Words(np.random.default_rng(6), ["the", "Of", "inter", "x9"]), n)
     assert len(text.encode()) == n
     check(name, text, n)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_whitespace_runs_across_words(name):
+    """Whitespace runs with CR/LF that reach one or more 64-byte words past
+    the character asking about them, at every alignment, ended by letters,
+    punctuation, non-ASCII characters and whitespace, the text's end, and
+    (as documents of one batch) a document's start."""
+    rng = np.random.default_rng(72)
+    unit = ["\n", "\r\n", "\r", "\t", " ", "　", "é", "a", "!", "！", "1", "中"]
+    docs = []
+    for k in range(160):
+        s = "x" * (k % 67)
+        for _ in range(int(rng.integers(1, 14))):
+            if rng.random() < 0.4:
+                s += " " * int(rng.integers(1, 150))
+            else:
+                s += unit[int(rng.integers(0, len(unit)))] * int(rng.integers(1, 4))
+        docs.append(s)
+    check(name, "".join(docs), "joined")
+    for k, (d, got) in enumerate(zip(docs, tok(name).encode_batch(docs))):
+        assert np.array_equal(got.array, kit(name).expected(d)), (name, k)

@@ -389,10 +389,11 @@ __device__ __forceinline__ uint64_t nrun_load(const uint64_t* p) {
 }
 constexpr int PT_HALO = 64;
 constexpr int PT_PAD = 80;  // >= PT_HALO + 4, a multiple of 16
-// the staged sizes of a tile of TILE bytes: entries, bytes, and doc-mask
-// words from tile word - 3
+// the staged sizes of a tile of TILE bytes: entries, bytes (the word after
+// the tile has its own next word's bytes too), and doc-mask words from tile
+// word - 3
 constexpr int pt_span(int tile) { return tile + 2 * PT_HALO; }
-constexpr int pt_bytes(int tile) { return tile + 2 * PT_PAD; }
+constexpr int pt_bytes(int tile) { return tile + 2 * PT_PAD + 64; }
 constexpr int pt_dmw(int tile) { return tile / 64 + 6; }
 
 // LCtx answers from a block's LDS tile and falls back to GCtx for
@@ -1605,6 +1606,27 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       const bool open = lead && !d0 && r < 0;
       int64_t far = -1;  // (deepseek) FAST_FAR: where the search starts
       if (__builtin_amdgcn_ballot_w64(open)) {  // wave-uniform
+        // The byte kinds of the words beside this one, where a whitespace
+        // run that a CR/LF case asks about reaches past the word's edge
+        // (wave-uniform: an indented line's run crosses one every few
+        // lines, and a walk along it, a character a step and past the
+        // staged bytes from HBM, held the whole tile up: 4,194,304 chars of
+        // code took 134 us here, 75 with these masks; 20,011 chars 41 -> 17).
+        uint64_t nWS = 0, nCR = 0, nHI = 0, pWS = 0, pCR = 0, pHI = 0;
+        if (__builtin_amdgcn_ballot_w64(open && r == FAST_CRLF)) {
+          if ((mWS | mCR) >> 63) {
+            const uint32_t b = sb[sj + 64];
+            nWS = __ballot(b == ' ' || b == '\t' || b == 0x0B || b == 0x0C);
+            nCR = __ballot(b == '\n' || b == '\r');
+            nHI = __ballot(b >= 0x80);
+          }
+          if (mCR & 1) {
+            const uint32_t b = sb[sj - 64];
+            pWS = __ballot(b == ' ' || b == '\t' || b == 0x0B || b == 0x0C);
+            pCR = __ballot(b == '\n' || b == '\r');
+            pHI = __ballot(b >= 0x80);
+          }
+        }
         if (open) {
           const uint64_t below = (1ULL << lane) - 1;
           // document starts in this word (a run ends at one, as at the
@@ -1624,28 +1646,40 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
             }
             r = cnt % (uint32_t)t.dmax == 0;
           } else if (r == FAST_CRLF && bb < 0x80) {
-            // another CR/LF ahead in the run: it shows in the word before
-            // the first byte that is neither (unless that byte is not
-            // ASCII) and before the next document start
+            // another CR/LF ahead in the run: it shows before the first
+            // byte that is neither (unless that byte is not ASCII) and
+            // before the next document start, in this word or the next
             const uint64_t above = ~mask_le(lane);
             const uint64_t stop = ~(mWS | mCR) & above;
-            const int f = stop ? __builtin_ctzll(stop) : 64;
-            const int fd = (dmw & above) ? __builtin_ctzll(dmw & above) : 64;
-            const int g = (mCR & above) ? __builtin_ctzll(mCR & above) : 64;
+            int f = stop ? __builtin_ctzll(stop) : 64;
+            int fd = (dmw & above) ? __builtin_ctzll(dmw & above) : 64;
+            int g = (mCR & above) ? __builtin_ctzll(mCR & above) : 64;
+            if (f == 64 && fd == 64 && g == 64) {
+              const uint64_t dmn = D ? sdm[wd + 1 - wlo] : 0;
+              f = ~(nWS | nCR) ? 64 + __builtin_ctzll(~(nWS | nCR)) : 128;
+              fd = dmn ? 64 + __builtin_ctzll(dmn) : 128;
+              g = nCR ? 64 + __builtin_ctzll(nCR) : 128;
+            }
+            const bool hi = f < 64 ? (mHI >> f) & 1 : f == 128 || ((nHI >> (f - 64)) & 1);
             if (g < f && g < fd) {
               // then the char before the CR/LF run that precedes i (none
-              // when a document starts inside that run)
+              // when a document starts inside that run, or the text does)
               const uint64_t nc = ~mCR & below;
               const int h = nc ? 63 - __builtin_clzll(nc) : -1;
-              if (dmw & lanes_in(h + 1, lane)) {
+              if ((dmw & lanes_in(h + 1, lane)) || (h < 0 && wd == 0)) {
                 r = 0;
               } else if (h >= 0) {
                 if ((mWS >> h) & 1) r = 0;
                 else if (!((mHI >> h) & 1)) r = kcl(se[Li - (lane - h)]) == KP;
+              } else if (~pCR) {
+                const int q = 63 - __builtin_clzll(~pCR);  // in the word before
+                const uint64_t dmp = D ? sdm[wd - 1 - wlo] : 0;
+                if ((dmp & lanes_in(q + 1, 64)) || ((pWS >> q) & 1)) r = 0;
+                else if (!((pHI >> q) & 1)) r = kcl(se[Li - lane - 64 + q]) == KP;
               }
-            } else if (fd < 64 && fd <= f) {
+            } else if (fd <= f && fd != 64 && fd < 128) {
               r = 1;
-            } else if (f < 64 && !((mHI >> f) & 1)) {
+            } else if (!hi) {
               r = 1;
             }
           } else if (RS == RS_DEEPSEEK && r == FAST_GENERAL) {
@@ -1771,14 +1805,28 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
         const uint64_t mHI = __ballot(bb >= 0x80);
         const uint64_t above = ~mask_le(lane);
         const uint64_t stop = ~(mWS | mCR) & above;
-        const int fs = stop ? __builtin_ctzll(stop) : 64;
+        int fs = stop ? __builtin_ctzll(stop) : 64;
         const uint64_t dmw = D ? sdm[(base >> 6) + k - wlo] & above : 0;
-        const int fd = dmw ? __builtin_ctzll(dmw) : 64;
-        const int gc = (mCR & above) ? __builtin_ctzll(mCR & above) : 64;
+        int fd = dmw ? __builtin_ctzll(dmw) : 64;
+        int gc = (mCR & above) ? __builtin_ctzll(mCR & above) : 64;
+        bool hi = fs < 64 && ((mHI >> fs) & 1);
+        if ((mWS | mCR) >> 63) {  // (wave-uniform) the run goes on in the next word
+          const uint32_t b = sb[64 * (k + 1) + lane + PT_PAD];
+          const uint64_t nWS = __ballot(b == ' ' || b == '\t' || b == 0x0B || b == 0x0C);
+          const uint64_t nCR = __ballot(b == '\n' || b == '\r');
+          const uint64_t nHI = __ballot(b >= 0x80);
+          if (fs == 64 && fd == 64 && gc == 64) {
+            const uint64_t ns = ~(nWS | nCR), dmn = D ? sdm[(base >> 6) + k + 1 - wlo] : 0;
+            fs = ns ? 64 + __builtin_ctzll(ns) : 128;
+            fd = dmn ? 64 + __builtin_ctzll(dmn) : 128;
+            gc = nCR ? 64 + __builtin_ctzll(nCR) : 128;
+            hi = ns == 0 || ((nHI >> (fs & 63)) & 1);
+          }
+        }
         const int end = fd < fs ? fd : fs;  // the run's end, as far as the masks go
         if (gc < end) ws_hint = 0;
-        else if (fd <= fs && fd < 64) ws_hint = 1;
-        else if (fs < 64 && !((mHI >> fs) & 1)) ws_hint = 1;
+        else if (fd <= fs && fd != 64 && fd < 128) ws_hint = 1;
+        else if (fs != 64 && !hi) ws_hint = 1;
       }
       *f = o2_ident<W>();
       *g = 0;
