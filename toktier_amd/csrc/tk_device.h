@@ -50,6 +50,27 @@ __host__ __device__ __forceinline__ uint32_t pair_alt(uint32_t b1, uint32_t tag,
   return (b1 ^ (h >> (32 - bits))) & ((1u << bits) - 1);
 }
 
+// Seams: positions inside a piece that no merge can cross, so the piece's
+// BPE is the BPE of its parts (k_piece_split cuts pieces there). A symbol that
+// spans a position spells some token (a rule's product, or a vocabulary
+// entry), so a position is a seam when no token, laid over the text around
+// it, agrees with the bytes next to it. What the tokens hold across each of
+// their inner positions is kept as keys of SEAM_CTX bytes a side, or fewer
+// where the token begins or ends there: type (A - 1) * SEAM_CTX + (B - 1) for
+// A bytes before and B after. seam_mask[last byte before << 8 | first byte
+// after] has a bit per type that occurs with that byte pair; seam_bits is a
+// one-hash bitmap of the keys (a false bit only loses a seam). One byte more
+// of context changes little (pieces of 65-512 bytes of the CJK workload: 22%
+// of their bytes stay in parts over 64 bytes with 4 bytes a side, 22% with 6
+// and with the whole tokens; 30% with 3).
+constexpr int SEAM_CTX = 4;
+__host__ __device__ __forceinline__ uint32_t seam_hash(uint32_t left, uint32_t right,
+                                                       uint32_t type) {
+  uint32_t h = left * 0x9E3779B1u + right * 0x85EBCA77u + type * 0x27D4EB2Fu;
+  h ^= h >> 15;
+  return h * 0x2C1B3C6Du;
+}
+
 // Device copies of the family tables, in the engine's own layout.
 struct DevTables {
   const uint8_t* cls;          // [0x110000] P/L/N/S (deepseek: O L M N PS WS CRLF;
@@ -85,7 +106,34 @@ struct DevTables {
   // it before the table in HBM; nullptr: none
   const uint64_t* hot;
   uint32_t hot_k;
+  // seams (nullptr: pieces are not cut)
+  const uint16_t* seam_mask;   // [65536] key types by the byte pair
+  const uint32_t* seam_bits;   // key bitmap, bit seam_hash >> seam_shift
+  uint32_t seam_shift;
 };
+
+// k_bpe_mid packs a symbol, its pair's rank and its product in 64 bits, and
+// takes tables whose every byte has an id and whose rules fit the compact one
+__host__ __device__ __forceinline__ bool mid_table(const DevTables& t) {
+  return t.all_bytes && t.ctab;
+}
+
+// Parts of the queued pieces, by length (k_piece_split): up to 8, 16, 32, 64
+// and 128 bytes, and longer. A part is two words, its start | PART_SUB where
+// the piece was cut (the whole-piece vocabulary rule does not hold for a
+// part) and its end; the list of class c starts part_off(c, cap) parts into
+// DevWork::parts.
+constexpr int PART_CLASSES = 6, PART_LONG = 5, PART_MID = 3;
+constexpr uint32_t PART_SUB = 1u << 31;
+__host__ __device__ constexpr uint32_t part_max(int c) { return 8u << c; }
+__host__ __device__ inline size_t part_room(int c, size_t cap) {  // bytes disjoint
+  return c == 0 ? cap + 1 : cap / (part_max(c - 1) + 1) + 1;
+}
+__host__ __device__ inline size_t part_off(int c, size_t cap) {
+  size_t n = 0;
+  for (int q = 0; q < c; ++q) n += part_room(q, cap);
+  return n;
+}
 
 // The hot-pair table: 2^HOT_BITS buckets of 16 bytes (16 KB), the compact
 // table's bijection, bucket pair and slot layout with a 26-bit tag. An
@@ -120,7 +168,9 @@ struct DevWork {
   uint32_t out_cap;      // capacity of out in ids
   // long-piece segmentation (one bit / slot per byte)
   uint64_t* inlong;      // bytes of pieces over 64 bytes
-  uint64_t* cuts;        // candidate segment starts inside long pieces
+  uint64_t* cuts;        // segment starts inside long pieces: the seams, and
+                         // candidates, each certified
+  uint64_t* sure;        // the seams among them (words with bits in inlong)
   uint64_t* failm;       // cuts whose certificate failed this pass
   uint64_t* hfirst;      // first-token merge events, at the segment start
                          // (cert 2: every merge round, see HR_FIRST)
@@ -151,6 +201,10 @@ struct DevWork {
   uint32_t* vlist;       // the grid windows with long-piece bytes (k_win_list)
   uint32_t* vcount;      // their number (ctrl)
   uint32_t* nwide;       // queued pieces of 257..WIDE_MAX bytes (ctrl)
+  uint2* parts;          // the parts of the queued pieces, by class
+  uint64_t parts_cap;    // bytes the workspace holds (part_off)
+  uint32_t* npart;       // parts per class, then k_bpe_mid's unit counter, a
+                         // line each (ctrl)
   uint32_t* prepdone;    // k_bpe_pack waves done with the long pieces (ctrl)
   uint32_t* gate;        // GATE_WORDS in host memory, or nullptr
   uint32_t seq;          // call number written to gate[GATE_SEQ]
@@ -185,22 +239,26 @@ constexpr uint64_t HR_FIRST = 1ull << 31, HR_LAST = 1ull << 30;
 // ctrl word layout (device -> host)
 // (the words of segment x of the piece lists start at CTRL_PSEG + x *
 // CTRL_PSEG_STRIDE: k_bpe_pack's unit counter, then on the next 128-byte
-// line the pieces listed per class, at CTRL_PSEG_COUNT + class)
+// line the pieces listed per class, at CTRL_PSEG_COUNT + class; then, a
+// 128-byte line each, the parts per class and k_bpe_mid's unit counter:
+// updates of one line are taken one after another, ~40 ns each)
 constexpr int CTRL_STATUS = 0, CTRL_TOTAL = 1, CTRL_LONG = 2, CTRL_SEG = 3,
               CTRL_FAIL = 4, CTRL_BIG = 5, CTRL_NLIT = 6, CTRL_PASS = 7,
               CTRL_FAIL2 = 8, CTRL_PREP = 9, CTRL_WIDE = 10, CTRL_ROWS = 11,
               CTRL_WIN = 12, CTRL_ROWQ = 16,  // (ROWQ: PACK_XCDS words)
               CTRL_VLIST = 24,
               CTRL_PSEG = 64, CTRL_PSEG_STRIDE = 64,
-              CTRL_PSEG_COUNT = 32, CTRL_WORDS = CTRL_PSEG + 8 * CTRL_PSEG_STRIDE;
+              CTRL_PSEG_COUNT = 32, CTRL_PART = CTRL_PSEG + 8 * CTRL_PSEG_STRIDE,
+              CTRL_PART_STRIDE = 32, CTRL_WORDS = CTRL_PART + 7 * CTRL_PART_STRIDE;
 // gate words in host memory: k_bpe_pack writes GATE_NLONG / GATE_NROWS /
-// GATE_NWIDE / GATE_BIG and then GATE_SEQ (the host learns, while the packed merge runs,
+// GATE_NWIDE / GATE_BIG / GATE_NMID and then GATE_SEQ (the host learns, while the packed merge runs,
 // whether the side streams' long-piece stages have any work), k_compact's
 // last block writes the request's outcome (status, id count, failed cuts)
 // and then GATE_DONE, so no copy is needed to read it
 constexpr int GATE_SEQ = 0, GATE_BIG = 1, GATE_STATUS = 2, GATE_TOTAL = 3,
               GATE_FAIL = 4, GATE_DONE = 5, GATE_NLONG = 6, GATE_NLIT = 7,
-              GATE_PASS = 8, GATE_NWIDE = 9, GATE_NROWS = 10, GATE_WORDS = 16;
+              GATE_PASS = 8, GATE_NWIDE = 9, GATE_NROWS = 10, GATE_NMID = 11,
+              GATE_WORDS = 16;
 
 // Added-token literals on the device: the trie over their bytes, stored as
 // one hash table of its edges. Slot = key << 36 | child << 16 | term, key =
@@ -236,15 +294,22 @@ __host__ __device__ __forceinline__ uint32_t added_slot(uint32_t key,
 // side streams' long-piece kernels, which run beside it
 constexpr int PACK_BLOCKS = 1792;
 // k_bpe_pack merges the queued pieces of 65..128 bytes itself when at most
-// this many pieces over 64 bytes are queued; else k_bpe_rows does
+// this many pieces over 64 bytes are queued; else k_piece_split and
+// k_bpe_mid do (k_bpe_rows, for tables that those do not take)
 constexpr int PACK_ROWS_MAX = 8192;
+// k_bpe_pack merges the pieces of 33..64 bytes (class PACK_MID), one a wave,
+// when there are at most this many; else k_bpe_mid does, one a lane
+constexpr int PACK_MID_MAX = 4096;
+constexpr int PACK_MID = PACK_CLASSES - 1;
 // The piece lists come in PACK_XCDS segments: segment x holds the pieces of
 // the k_pretok tiles b with b % PACK_XCDS == x (those of one XCD: workgroups
 // go to the XCDs in turn), and the k_bpe_pack blocks of the same residue
 // merge them, each XCD's units handed out by a counter of its own
 constexpr int PACK_XCDS = 8;
-static_assert(CTRL_WORDS == CTRL_PSEG + PACK_XCDS * CTRL_PSEG_STRIDE,
+static_assert(CTRL_PART == CTRL_PSEG + PACK_XCDS * CTRL_PSEG_STRIDE,
               "one control line per segment");
+static_assert(CTRL_WORDS == CTRL_PART + (PART_CLASSES + 1) * CTRL_PART_STRIDE,
+              "a line per part class and one for the unit counter");
 static_assert(CTRL_ROWQ + PACK_XCDS <= CTRL_VLIST, "row counters before the window list's");
 static_assert(CTRL_VLIST < CTRL_PSEG, "the window count before the segment lines");
 // k_bpe_pack's blocks for nb bytes: a wave per work unit of a segment (one
@@ -345,11 +410,19 @@ hipError_t launch_pretok(const DevTables& t, const DevWork& w, hipStream_t s,
                          hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
 hipError_t launch_bpe_pack(const DevTables& t, const DevWork& w, hipStream_t s,
                            hipEvent_t start, hipEvent_t stop);
+// the parts of the nlong queued pieces of 65..WIDE_MAX bytes, by class
+hipError_t launch_piece_split(const DevTables& t, const DevWork& w, hipStream_t s,
+                              uint32_t nlong);
+// the parts of up to 128 bytes (split), and the nmid listed pieces of 33..64
+// bytes (0: none), one a lane
+hipError_t launch_bpe_mid(const DevTables& t, const DevWork& w, hipStream_t s,
+                          bool split, uint32_t nmid);
+// split: the parts over 128 bytes instead of the queued pieces
 hipError_t launch_bpe_rows(const DevTables& t, const DevWork& w, hipStream_t s,
-                           uint32_t nlong, hipEvent_t start = nullptr,
+                           uint32_t nlong, bool split, hipEvent_t start = nullptr,
                            hipEvent_t stop = nullptr);
 hipError_t launch_bpe_wide(const DevTables& t, const DevWork& w, hipStream_t s,
-                           hipEvent_t stop, uint32_t nlong);
+                           hipEvent_t stop, uint32_t nlong, bool split);
 hipError_t launch_long_windows(const DevTables& t, const DevWork& w,
                                hipStream_t s, hipEvent_t start = nullptr,
                                hipEvent_t stop = nullptr);

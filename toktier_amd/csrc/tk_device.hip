@@ -2736,7 +2736,14 @@ void k_bpe_pack(DevTables t, DevWork w) {
   uint32_t nl = *w.longcount;  // queued long pieces
   if (nl > w.long_cap) nl = w.long_cap;
   if (wv == 0) {
-    const uint32_t cnt = cl ? seg[CTRL_PSEG_COUNT + lane] : 0u;
+    uint32_t cnt = cl ? seg[CTRL_PSEG_COUNT + lane] : 0u;
+    // (more than PACK_MID_MAX pieces of 33..64 bytes go to k_bpe_mid)
+    const uint32_t mid = wave_incl_scan(
+        lane < PACK_XCDS ? w.pseg[lane * CTRL_PSEG_STRIDE + CTRL_PSEG_COUNT + PACK_MID] : 0u,
+        lane);
+    if (lane == PACK_MID && mid_table(t) &&
+        __builtin_amdgcn_readlane((int)mid, PACK_XCDS - 1) > PACK_MID_MAX)
+      cnt = 0;
     const uint32_t geo = cl ? PACK_GEO[lane] : 0u;
     const uint32_t per = cl ? (geo >> 8) & 0xFF : 1u;
     const uint32_t nu = (cnt + per - 1) / per;  // the class's units
@@ -2792,6 +2799,11 @@ void k_bpe_pack(DevTables t, DevWork w) {
                                                  __HIP_MEMORY_SCOPE_AGENT);
           w.gate[GATE_NWIDE] = __hip_atomic_load(w.nwide, __ATOMIC_RELAXED,
                                                  __HIP_MEMORY_SCOPE_AGENT);
+          uint32_t mid = 0;
+#pragma unroll
+          for (int q = 0; q < PACK_XCDS; ++q)
+            mid += w.pseg[q * CTRL_PSEG_STRIDE + CTRL_PSEG_COUNT + PACK_MID];
+          w.gate[GATE_NMID] = mid;
           w.gate[GATE_BIG] = __hip_atomic_load(w.nbig, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT);
           __threadfence_system();
@@ -3219,7 +3231,7 @@ __device__ __forceinline__ uint64_t wide_pair(const DevTables& t,
   return pair_lookup(t, x & ~SYM_RAW, y & ~SYM_RAW);
 }
 
-__device__ void wave_bpe_wide(const DevTables& t, const DevWork& w,
+__device__ __forceinline__ void wave_bpe_wide(const DevTables& t, const DevWork& w,
                               uint32_t a, int len, bool vocab_first,
                               bool hist, WideLds& L) {
   const int lane = threadIdx.x & 63;
@@ -3678,6 +3690,329 @@ __device__ __forceinline__ void wave_bpe_rows(const DevTables& t,
   if (H && lane == 0) w.hmeta[a] = t.cert == 2 ? nfirst : nfirst | (nlast << 16);
 }
 
+// One piece of n <= N bytes per lane (n == 0: none), merged serially by its
+// lane in the HF order, as lane_bpe does, with the state in LDS (L: this
+// wave's mid_words(N) words), position p of lane l at [p][l], so that a wave's
+// accesses never meet in a bank whatever positions its lanes are at: a word
+// rank << 13 | symbol's low 13 bits, a word product << 5 | symbol's high 5
+// bits (mid_table: ids below 2^18, ranks below 2^19 - 1; rank MID_NONE: no
+// rule, or not live), and per 8 positions the lowest rank << 7 | position. A
+// step takes the lowest of the N / 8 minima, looks the two changed pairs up
+// and takes the minima of the changed positions' chunks anew. A wave step
+// merges 64 pairs where one piece a wave merges one (or the occurrences of
+// one rank); its ~200 vector instructions and two lookups take ~2,000 cycles
+// with one or two waves a SIMD.
+constexpr uint32_t MID_NONE = 0x7FFFFu;
+__host__ __device__ constexpr int mid_words(int n) { return (2 * n + n / 8) * 64; }
+template <int N>
+__device__ __forceinline__ void lane_bpe_lds(const DevTables& t, const DevWork& w,
+                                             uint32_t* L, int64_t a, int n, bool whole, int lane) {
+  constexpr int W = (N + 63) / 64;
+  static_assert(N == 32 || N == 64 || N == 128, "live masks of one or two words");
+  uint32_t* const lo = L + lane;                   // [p * 64]
+  uint32_t* const hi = L + N * 64 + lane;          // [p * 64]
+  uint32_t* const cm = L + 2 * N * 64 + lane;      // [chunk * 64]
+  if (n > 0 && t.ignore_merges && whole) {
+    // whole-piece vocabulary hit first (pretok_kernel.cu:921-943 role)
+    const int32_t hit = vocab_lookup(t, w.text + a, n);
+    if (hit >= 0) {
+      for (int i = 0; i < n; ++i) w.tok[a + i] = i == 0 ? (uint32_t)hit : INVALID_ID;
+      n = 0;
+    }
+  }
+  uint64_t live[W];
+#pragma unroll
+  for (int k = 0; k < W; ++k)
+    live[k] = n >= 64 * (k + 1) ? ~0ULL : n > 64 * k ? (1ULL << (n - 64 * k)) - 1 : 0ULL;
+  uint32_t nmax = (uint32_t)n;  // the wave's longest piece
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, d));
+  const int chunks = (__builtin_amdgcn_readfirstlane((int)nmax) + 7) / 8;
+  for (int c = 0; c < chunks; ++c) {
+    uint32_t by[9];
+#pragma unroll
+    for (int j = 0; j < 9; ++j) by[j] = 8 * c + j < n ? w.text[a + 8 * c + j] : 0u;
+    uint64_t v[8];
+    uint32_t sy[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      v[j] = 8 * c + j + 1 < n ? t.bytepair[(by[j] << 8) | by[j + 1]] : ~0ULL;
+      sy[j] = (uint32_t)t.byte_id[by[j]];
+    }
+    uint32_t m = RANK_INF;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t r = v[j] == ~0ULL ? MID_NONE : (uint32_t)(v[j] >> 32);
+      lo[(8 * c + j) * 64] = r << 13 | (sy[j] & 0x1FFF);
+      hi[(8 * c + j) * 64] = ((uint32_t)v[j] & 0x3FFFF) << 5 | sy[j] >> 13;
+      m = min(m, r << 7 | (uint32_t)(8 * c + j));
+    }
+    cm[c * 64] = m;
+  }
+  for (int c = chunks; c < N / 8; ++c) cm[c * 64] = RANK_INF;
+  for (;;) {
+    uint32_t best = RANK_INF;
+#pragma unroll
+    for (int c = 0; c < N / 8; ++c) best = min(best, cm[c * 64]);
+    if (best >= MID_NONE << 7) break;  // this lane's piece is finished
+    // bi absorbs the next live position nb; p and nn: its live neighbours
+    // after the merge (-1: none)
+    const int bi = (int)(best & 127);
+    auto next = [&](int q) {
+      if (W == 1) {
+        const uint64_t m = live[0] & (~1ULL << q);
+        return m ? __builtin_ctzll(m) : -1;
+      }
+      const uint64_t m0 = q < 64 ? live[0] & (~1ULL << (q & 63)) : 0ULL;
+      const uint64_t m1 = q < 64 ? live[W - 1] : live[W - 1] & (~1ULL << (q & 63));
+      return m0 ? __builtin_ctzll(m0) : m1 ? 64 + __builtin_ctzll(m1) : -1;
+    };
+    const int nb = next(bi);
+    const int nn = next(nb);
+    int p;
+    {
+      const uint64_t below = (1ULL << (bi & 63)) - 1;
+      const uint64_t m0 = bi < 64 ? live[0] & below : live[0];
+      const uint64_t m1 = W == 2 && bi >= 64 ? live[W - 1] & below : 0ULL;
+      p = m1 ? 127 - __builtin_clzll(m1) : m0 ? 63 - __builtin_clzll(m0) : -1;
+    }
+    if (W == 1 || nb < 64) live[0] &= ~(1ULL << (nb & 63));
+    else live[W - 1] &= ~(1ULL << (nb & 63));
+    const int ps = p < 0 ? bi : p, ns = nn < 0 ? bi : nn;
+    const uint32_t mid = hi[bi * 64] >> 5;
+    const uint32_t sp = (lo[ps * 64] & 0x1FFF) | (hi[ps * 64] & 31) << 13;
+    const uint32_t sn = (lo[ns * 64] & 0x1FFF) | (hi[ns * 64] & 31) << 13;
+    uint32_t rp = MID_NONE, mp = 0, rb = MID_NONE, mb = 0, r_, m_;
+    if (p >= 0 && ctab_find(t, sp, mid, &r_, &m_)) {
+      rp = r_;
+      mp = m_;
+    }
+    if (nn >= 0 && ctab_find(t, mid, sn, &r_, &m_)) {
+      rb = r_;
+      mb = m_;
+    }
+    lo[nb * 64] = MID_NONE << 13;
+    lo[bi * 64] = rb << 13 | (mid & 0x1FFF);
+    hi[bi * 64] = mb << 5 | mid >> 13;
+    if (p >= 0) {
+      lo[p * 64] = rp << 13 | (sp & 0x1FFF);
+      hi[p * 64] = mp << 5 | sp >> 13;
+    }
+    // the minima of the changed positions' chunks, their reads all issued
+    // before any is used (one LDS round trip)
+    const int c0 = bi >> 3, c1 = nb >> 3, c2 = ps >> 3;
+    uint32_t k0[8], k1[8], k2[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      k0[j] = lo[(8 * c0 + j) * 64];
+      k1[j] = lo[(8 * c1 + j) * 64];
+      k2[j] = lo[(8 * c2 + j) * 64];
+    }
+    uint32_t m0 = RANK_INF, m1 = RANK_INF, m2 = RANK_INF;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      m0 = min(m0, k0[j] >> 13 << 7 | (uint32_t)(8 * c0 + j));
+      m1 = min(m1, k1[j] >> 13 << 7 | (uint32_t)(8 * c1 + j));
+      m2 = min(m2, k2[j] >> 13 << 7 | (uint32_t)(8 * c2 + j));
+    }
+    cm[c0 * 64] = m0;
+    cm[c1 * 64] = m1;
+    cm[c2 * 64] = m2;
+  }
+#pragma unroll 8
+  for (int i = 0; i < 8 * chunks; ++i) {
+    const uint32_t sy = (lo[i * 64] & 0x1FFF) | (hi[i * 64] & 31) << 13;
+    const uint64_t lv = W == 2 && i >= 64 ? live[W - 1] : live[0];
+    if (i < n) w.tok[a + i] = ((lv >> (i & 63)) & 1) ? sy : INVALID_ID;
+  }
+}
+
+// The queued pieces of 65..WIDE_MAX bytes cut at their seams (tk_device.h) and
+// their parts listed by length, 32 pieces a block. A CJK sentence is one
+// piece of 12-180 bytes, whose merge by a wave is a chain of ~50 dependent
+// rounds; its parts, mostly of a few bytes, are merged one a lane
+// (k_bpe_mid). Per piece a wave takes 64 positions at a time, a lane each: a
+// position inside a character, or one that is inside a two-byte token
+// whatever its context, is none at once, one with no key type for its byte
+// pair is a seam at once, and the others probe their types' keys one after
+// another (one to six dependent loads: the kernel's time is their latency).
+constexpr int SPLIT_PIECES = 32, SPLIT_TPB = 512;
+// Is there a seam between the bytes left (nearest lowest) and right? m: the
+// key types to probe (seam_types).
+__device__ __forceinline__ bool seam_probe(const DevTables& t, uint32_t left,
+                                           uint32_t right, uint32_t m) {
+  bool hit = m & 1;
+  for (; m && !hit; m &= m - 1) {
+    const uint32_t type = (uint32_t)__builtin_ctz(m);
+    const uint32_t h = seam_hash(left & (~0u >> (24 - 8 * (type / SEAM_CTX))),
+                                 right & (~0u >> (24 - 8 * (type % SEAM_CTX))), type) >>
+                       t.seam_shift;
+    hit = (t.seam_bits[h >> 5] >> (h & 31)) & 1;
+  }
+  return !hit;
+}
+// The bytes around x[0] with `before` of them ahead of it and `after` from it
+// on (at least one each), and the key types that leaves room for.
+__device__ __forceinline__ uint32_t seam_types(const DevTables& t, const uint8_t* x,
+                                               int64_t before, int64_t after,
+                                               uint32_t* left, uint32_t* right) {
+  uint32_t l = 0, r = 0;
+#pragma unroll
+  for (int j = 0; j < SEAM_CTX; ++j) {
+    if (j < before) l |= (uint32_t)x[-1 - j] << (8 * j);
+    if (j < after) r |= (uint32_t)x[j] << (8 * j);
+  }
+  uint32_t m = t.seam_mask[(l & 0xFF) << 8 | (r & 0xFF)];
+  if (before < SEAM_CTX) m &= (1u << (SEAM_CTX * before)) - 1;
+  if (after < SEAM_CTX) m &= 0x1111u * ((1u << after) - 1);
+  *left = l;
+  *right = r;
+  return m;
+}
+__device__ __forceinline__ uint32_t part_count(const DevWork& w, int c) {
+  return w.npart[c * CTRL_PART_STRIDE];
+}
+__global__ __launch_bounds__(SPLIT_TPB) void k_piece_split(DevTables t, DevWork w) {
+  constexpr int WORDS = WIDE_MAX / 64;
+  static_assert(SPLIT_PIECES * WORDS <= SPLIT_TPB, "a thread per piece and word");
+  __shared__ uint32_t sa[SPLIT_PIECES], sl[SPLIT_PIECES];
+  __shared__ uint64_t sm[SPLIT_PIECES][WORDS];  // seams (bit 0: the piece's start)
+  __shared__ uint32_t cnt[PART_CLASSES], at[PART_CLASSES];
+  const int tid = threadIdx.x, lane = tid & 63, wv = wave_id();
+  if (tid < PART_CLASSES) cnt[tid] = 0;
+  uint32_t n = *w.longcount;
+  if (n > w.long_cap) n = w.long_cap;
+  const uint8_t* const x = w.text;
+  for (int e = wv; e < SPLIT_PIECES; e += SPLIT_TPB / 64) {
+    const uint32_t k = blockIdx.x * SPLIT_PIECES + e;
+    uint32_t a = 0, len = 0;
+    if (k < n) {
+      a = w.longlist[2 * k];
+      len = w.longlist[2 * k + 1] - a;
+      if (len > (uint32_t)WIDE_MAX) len = 0;  // (cut and certified)
+    }
+    a = (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+    len = (uint32_t)__builtin_amdgcn_readfirstlane((int)len);
+    if (lane == 0) {
+      sa[e] = a;
+      sl[e] = len;
+    }
+    for (int c = 0; c < WORDS && 64u * c < len; ++c) {
+      const int i = 64 * c + lane;  // bytes of the piece before the position
+      uint32_t m = 1, left = 0, right = 0;
+      if (t.seam_mask && i > 0 && i < (int)len && !is_cont(x[a + i]))
+        m = seam_types(t, x + a + i, i, (int)len - i, &left, &right);
+      const uint64_t cut = __ballot(seam_probe(t, left, right, m));
+      if (lane == 0) sm[e][c] = cut | (c == 0 ? 1 : 0);
+    }
+  }
+  __syncthreads();
+  // thread (piece, word): the parts that start in the word, counted, then
+  // listed (one counter update per class and block)
+  const int e = tid / WORDS % SPLIT_PIECES, c = tid % WORDS;
+  const uint32_t len = tid < SPLIT_PIECES * WORDS ? sl[e] : 0u;
+  const int words = (int)((len + 63) / 64);
+  const bool mine = c < words;
+  bool sub = false;
+  for (int q = 0; q < words; ++q) sub |= (q ? sm[e][q] : sm[e][q] & ~1ULL) != 0;
+  auto each = [&](auto fn) {
+    for (uint64_t m = mine ? sm[e][c] : 0; m; m &= m - 1) {
+      const uint32_t from = 64u * c + (uint32_t)__builtin_ctzll(m);
+      uint32_t to = len;
+      const uint64_t more = m & (m - 1);
+      if (more) {
+        to = 64u * c + (uint32_t)__builtin_ctzll(more);
+      } else {
+        for (int q = c + 1; q < words; ++q)
+          if (sm[e][q]) {
+            to = 64u * q + (uint32_t)__builtin_ctzll(sm[e][q]);
+            break;
+          }
+      }
+      int cls = 0;
+#pragma unroll
+      for (int q = 0; q < PART_LONG; ++q) cls += to - from > part_max(q);
+      fn(from, to, cls);
+    }
+  };
+  each([&](uint32_t, uint32_t, int cls) { atomicAdd(&cnt[cls], 1u); });
+  __syncthreads();
+  if (tid < PART_CLASSES) {
+    at[tid] = cnt[tid] ? atomicAdd(w.npart + tid * CTRL_PART_STRIDE, cnt[tid]) : 0u;
+    cnt[tid] = 0;
+  }
+  __syncthreads();
+  each([&](uint32_t from, uint32_t to, int cls) {
+    const uint32_t k = at[cls] + atomicAdd(&cnt[cls], 1u);
+    w.parts[part_off(cls, w.parts_cap) + k] =
+        make_uint2((sa[e] + from) | (sub ? PART_SUB : 0u), sa[e] + to);
+  });
+}
+
+// Parts (and, nmid set, the listed pieces of 33..64 bytes), one a lane, in
+// work units of one block each, longest first: 64 parts of 65..128 bytes (one
+// wave, all of the block's LDS), 128 of 33..64 (two waves, half of it each),
+// 256 shorter ones (four waves). Block b takes unit b first, every later one
+// from a counter.
+constexpr uint32_t MID_BLOCKS = 512;  // two of 69,632 bytes of LDS on every CU
+__global__ __launch_bounds__(256) void k_bpe_mid(DevTables t, DevWork w, int split, int nmid) {
+  __shared__ uint32_t lds[mid_words(128)];
+  static_assert(2 * mid_words(64) <= mid_words(128) && 4 * mid_words(32) <= mid_words(128),
+                "the waves' shares");
+  __shared__ uint32_t sunit;
+  const int lane = threadIdx.x & 63, wv = wave_id();
+  // the unit ranges, lane k: 0 parts of 65..128, 1 of 33..64, 2..9 the
+  // segments' lists of class PACK_MID, 10..12 the parts of up to 32, 16, 8
+  uint32_t cnt = 0, per = 1;
+  if (lane == 0) { cnt = split ? part_count(w, 4) : 0u; per = 64; }
+  else if (lane == 1) { cnt = split ? part_count(w, PART_MID) : 0u; per = 128; }
+  else if (lane < 2 + PACK_XCDS) {
+    cnt = nmid ? w.pseg[(lane - 2) * CTRL_PSEG_STRIDE + CTRL_PSEG_COUNT + PACK_MID] : 0u;
+    per = 128;
+  } else if (lane < 5 + PACK_XCDS) {
+    cnt = split ? part_count(w, 4 + PACK_XCDS - lane) : 0u;
+    per = 256;
+  }
+  const uint32_t units = (cnt + per - 1) / per, incl = wave_incl_scan(units, lane);
+  const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, 63);
+  for (uint32_t u = blockIdx.x; u < total;) {  // (block-uniform)
+    const uint32_t unit = u;
+    __syncthreads();  // (the last unit's LDS is free)
+    if (threadIdx.x == 0) sunit = gridDim.x + atomicAdd(w.npart + PART_CLASSES * CTRL_PART_STRIDE, 1u);
+    __syncthreads();
+    u = (uint32_t)__builtin_amdgcn_readfirstlane((int)sunit);
+    const int r = __builtin_ctzll(__ballot(incl > unit));
+    const uint32_t first = (unit - (uint32_t)__builtin_amdgcn_readlane((int)(incl - units), r)) *
+                           (uint32_t)__builtin_amdgcn_readlane((int)per, r);
+    const uint32_t end = (uint32_t)__builtin_amdgcn_readlane((int)cnt, r);
+    const int waves = r == 0 ? 1 : r < 2 + PACK_XCDS ? 2 : 4;
+    if (wv >= waves) continue;
+    const uint32_t k = first + 64 * wv + lane;
+    int64_t a = 0;
+    int n = 0;
+    bool whole = true;
+    if (k < end) {
+      if (r >= 2 && r < 2 + PACK_XCDS) {
+        const int tile = pretok_tile(w.nb);
+        const bool small = tile == PT_TILE_S;
+        a = w.plist[pack_seg_list((uint32_t)pretok_tiles(w.nb, tile), r - 2,
+                                  small ? PT_LOCAL_SLOTS_S : PT_LOCAL_SLOTS,
+                                  PACK_LOCAL_OFF[small][PACK_MID]) + k];
+        n = (int)(piece_end(w, a) - a);
+      } else {
+        const int cls = r == 0 ? 4 : r == 1 ? PART_MID : 4 + PACK_XCDS - r;
+        const uint2 v = w.parts[part_off(cls, w.parts_cap) + k];
+        a = v.x & ~PART_SUB;
+        n = (int)(v.y - (uint32_t)a);
+        whole = !(v.x & PART_SUB);
+      }
+    }
+    if (waves == 1) lane_bpe_lds<128>(t, w, lds, a, n, whole, lane);
+    else if (waves == 2) lane_bpe_lds<64>(t, w, lds + wv * mid_words(64), a, n, whole, lane);
+    else lane_bpe_lds<32>(t, w, lds + wv * mid_words(32), a, n, whole, lane);
+  }
+}
+
 // Entries of 65..WIDE_MAX bytes from a (start, end) list, one wave each.
 __global__ __launch_bounds__(256) void k_bpe_wide(DevTables t, DevWork w,
                                                   const uint32_t* list,
@@ -3695,11 +4030,11 @@ __global__ __launch_bounds__(256) void k_bpe_wide(DevTables t, DevWork w,
   // priority over the other side work.
   if (hist && blockIdx.x * 4 + wv < n) __builtin_amdgcn_s_setprio(3);
   for (uint32_t k = blockIdx.x * 4 + wv; k < n; k += waves) {
-    const uint32_t a = list[2 * k], b = list[2 * k + 1];
+    const uint32_t v = list[2 * k], a = v & ~PART_SUB, b = list[2 * k + 1];
     const int len = (int)(b - a);
     // (pieces of up to 256 bytes without histories: k_bpe_pack, k_bpe_rows)
     if (len <= (hist ? 64 : 256) || len > WIDE_MAX) continue;  // wave-uniform
-    wave_bpe_wide(t, w, a, len, !hist, hist != 0, lds[wv]);
+    wave_bpe_wide(t, w, a, len, !hist && v == a, hist != 0, lds[wv]);
   }
 }
 
@@ -3708,10 +4043,14 @@ __global__ __launch_bounds__(256) void k_bpe_wide(DevTables t, DevWork w,
 // bitmap of at most ROWS_UNSAFE_LDS words, the launch gives each block a
 // copy of it in LDS (one lookup per merge round).
 constexpr uint32_t ROWS_UNSAFE_LDS = 12288;
-__global__ __launch_bounds__(256) void k_bpe_rows(DevTables t, DevWork w) {
+__global__ __launch_bounds__(256) void k_bpe_rows(DevTables t, DevWork w, int split) {
   extern __shared__ __align__(16) uint32_t unsafe_lds[];
-  uint32_t n = *w.longcount;
-  if (n > w.long_cap) n = w.long_cap;
+  // the queued pieces, or (split) the parts over 128 bytes
+  uint32_t n = split ? part_count(w, PART_LONG) : *w.longcount;
+  if (!split && n > w.long_cap) n = w.long_cap;
+  const uint32_t* const list =
+      split ? reinterpret_cast<const uint32_t*>(w.parts + part_off(PART_LONG, w.parts_cap))
+            : w.longlist;
   const bool lds = t.unsafe && t.unsafe_words <= ROWS_UNSAFE_LDS;
   if (lds)
     for (uint32_t j = threadIdx.x; j < t.unsafe_words; j += 256)
@@ -3726,9 +4065,9 @@ __global__ __launch_bounds__(256) void k_bpe_rows(DevTables t, DevWork w) {
   const int lane = threadIdx.x & 63, wv = wave_id();
   // (no issue priority: the cut / segment / certify chain of the long
   // pieces takes it)
-  // (pieces of 65..128 bytes too when k_bpe_pack left them: more than
-  // PACK_ROWS_MAX queued)
-  const int lo = n > (uint32_t)PACK_ROWS_MAX ? 64 : 128;
+  // (pieces of 65..128 bytes too when k_bpe_pack left them, more than
+  // PACK_ROWS_MAX queued, and they were not split)
+  const int lo = !split && n > (uint32_t)PACK_ROWS_MAX ? 64 : 128;
   // The queue in X contiguous shares (X = PACK_XCDS, or the blocks when
   // fewer), share x to the blocks of residue x (the blocks go to the XCDs
   // in turn). Wave g of a share's G waves takes entry g first, every later
@@ -3743,11 +4082,11 @@ __global__ __launch_bounds__(256) void k_bpe_rows(DevTables t, DevWork w) {
   const uint32_t G = (gridDim.x - x + X - 1) / X * 4;
   uint32_t k = k0 + blockIdx.x / X * 4 + wv;
   while (k < k1) {
-    const uint32_t a = w.longlist[2 * k], b = w.longlist[2 * k + 1];
+    const uint32_t v = list[2 * k], a = v & ~PART_SUB, b = list[2 * k + 1];
     const int len = (int)(b - a);
     if (len > lo && len <= 256) {  // wave-uniform
-      if (len <= 128) wave_bpe_rows<2>(t, w, a, len, true, lds ? unsafe_lds : nullptr, hot);
-      else wave_bpe_rows<4>(t, w, a, len, true, lds ? unsafe_lds : nullptr, hot);
+      if (len <= 128) wave_bpe_rows<2>(t, w, a, len, v == a, lds ? unsafe_lds : nullptr, hot);
+      else wave_bpe_rows<4>(t, w, a, len, v == a, lds ? unsafe_lds : nullptr, hot);
     }
     uint32_t got = 0;
     if (lane == 0)
@@ -3788,41 +4127,84 @@ __global__ void k_win_list(DevWork w, int64_t nwin) {
   if (need) w.vlist[base + (uint32_t)__popcll(m & ((1ULL << lane) - 1))] = (uint32_t)v;
 }
 
+// The seams of the long pieces: wave i over listed word i, a lane each
+// position (as k_piece_split; a position near a piece's end probes the bytes
+// past it too, which only loses seams). They are cuts that need no
+// certificate: between them most stretches are a few bytes long, and only
+// those over 64 bytes are cut further by the windows below.
+__global__ __launch_bounds__(256) void k_long_seams(DevTables t, DevWork w) {
+  const uint32_t i = blockIdx.x * 4 + wave_id();
+  if (i >= *w.vcount) return;
+  __builtin_amdgcn_s_setprio(2);  // (the long pieces' chain: k_long_windows)
+  const int lane = threadIdx.x & 63;
+  const int64_t v = w.vlist[i], p = 64 * v + lane;
+  const uint64_t in = w.inlong[v] & ~w.starts[v];
+  uint32_t m = 1, left = 0, right = 0;
+  if (t.seam_mask && ((in >> lane) & 1) && !is_cont(w.text[p]))
+    m = seam_types(t, w.text + p, p, w.nb - p, &left, &right);  // (p > 0: not a start)
+  const uint64_t cut = __ballot(seam_probe(t, left, right, m));
+  if (lane == 0) w.sure[v] = cut;
+}
+
+__device__ __forceinline__ uint64_t sure_word(const DevWork& w, int64_t wd) {
+  return w.starts[wd] | (w.sure[wd] & w.inlong[wd]);
+}
+
 __device__ __forceinline__ void long_window(const DevTables& t, const DevWork& w,
                                             int64_t v, int64_t nwin) {
   const int lane = threadIdx.x & 63;
-  auto seg = [&](int64_t wd) { return w.starts[wd]; };
+  auto seg = [&](int64_t wd) { return wd < 0 ? ~0ULL : sure_word(w, wd); };
   uint16_t* cut16 = reinterpret_cast<uint16_t*>(w.cuts);
+  const uint16_t* sure16 = reinterpret_cast<const uint16_t*>(w.sure);
   for (int phase = (v == nwin ? 1 : 0); phase < 2; ++phase) {
     const uint64_t L = inlong_window(w, v, phase);
     if (L == 0) continue;  // wave-uniform
     const int64_t base = phase == 0 ? v * 64 : v * 64 - 32;
-    uint64_t S;
-    bool E;
-    window_bits(v, phase, seg, &S, &E);
-    S |= 1;  // the window start cuts whatever runs into it
-    const uint64_t le = S & mask_le(lane);
-    const int ps = 63 - __builtin_clzll(le);
-    const uint64_t gt = S & ~mask_le(lane);
-    const int pe = gt ? __builtin_ctzll(gt) : 64;
-    const bool elig = (L >> lane) & 1;
-    const uint64_t live =
-        wave_bpe<false, false, false>(t, w, base, base + lane, lane, elig, ps, pe);
+    // the boundaries in the window (S) and in the 64 bytes either side
+    const uint64_t b0 = seg(v - 1), b1 = seg(v), b2 = seg(v + 1);
+    uint64_t S, below, above;
+    if (phase == 0) {
+      S = b1;
+      below = b0;
+      above = b2;
+    } else {
+      S = (b0 >> 32) | (b1 << 32);
+      below = (seg(v - 2) >> 32) | (b0 << 32);
+      above = (b1 >> 32) | (b2 << 32);
+    }
+    // the lane's stretch between two of them: over 64 bytes?
+    const uint64_t sle = S & mask_le(lane), sgt = S & ~mask_le(lane);
+    const int back = sle ? lane - (63 - __builtin_clzll(sle))
+                   : below ? lane + 1 + __builtin_clzll(below) : 128;
+    const int fwd = sgt ? __builtin_ctzll(sgt) - lane
+                  : above ? 64 - lane + __builtin_ctzll(above) : 128;
+    const uint64_t far = __ballot(back + fwd > 64 && ((L >> lane) & 1)) & 0x0000FFFFFFFF0000ULL;
+    uint64_t live = 0;
+    if (far) {  // wave-uniform
+      S |= 1;  // the window start cuts whatever runs into it
+      const uint64_t le = S & mask_le(lane);
+      const int ps = 63 - __builtin_clzll(le);
+      const uint64_t gt = S & ~mask_le(lane);
+      const int pe = gt ? __builtin_ctzll(gt) : 64;
+      const bool elig = (L >> lane) & 1;
+      live = wave_bpe<false, false, false>(t, w, base, base + lane, lane, elig, ps, pe) & far;
+    }
     if (lane == 0) {
       if (phase == 0) {
-        cut16[4 * v + 1] = (uint16_t)(live >> 16);
-        cut16[4 * v + 2] = (uint16_t)(live >> 32);
+        cut16[4 * v + 1] = (uint16_t)(live >> 16) | sure16[4 * v + 1];
+        cut16[4 * v + 2] = (uint16_t)(live >> 32) | sure16[4 * v + 2];
       } else {
-        if (v > 0) cut16[4 * (v - 1) + 3] = (uint16_t)(live >> 16);
-        cut16[4 * v] = (uint16_t)(live >> 32);
+        if (v > 0) cut16[4 * (v - 1) + 3] = (uint16_t)(live >> 16) | sure16[4 * (v - 1) + 3];
+        cut16[4 * v] = (uint16_t)(live >> 32) | sure16[4 * v];
       }
     }
   }
 }
 
-// Cut selection: BPE of the long-piece bytes of every window, window edges
-// taken as cuts; the token starts in the window's central 32 bytes become
-// candidate cuts. Aligned window v owns bits 16..47 of word v, shifted
+// Cut selection: BPE of the long-piece bytes of every window that a stretch
+// of over 64 bytes between seams (or piece ends) reaches into, window edges
+// taken as cuts; the token starts of such stretches in the window's central
+// 32 bytes become candidate cuts, beside the seams. Aligned window v owns bits 16..47 of word v, shifted
 // window v owns bits 48..63 of word v-1 and 0..15 of word v. Wave i takes
 // listed window i.
 __global__ __launch_bounds__(256) void k_long_windows(DevTables t, DevWork w,
@@ -3855,15 +4237,15 @@ __device__ __forceinline__ bool word_dirty(const uint64_t* d, int64_t wd) {
 __device__ void fail_segment_cuts(const DevWork& w, int64_t a, int64_t b) {
   auto is_cut = [&](int64_t c) {
     const int64_t wd = c >> 6;
-    return ((w.cuts[wd] & w.inlong[wd] & ~w.starts[wd]) >> (c & 63)) & 1;
+    return ((w.cuts[wd] & w.inlong[wd] & ~sure_word(w, wd)) >> (c & 63)) & 1;
   };
   auto fail = [&](int64_t c) {
     atomicOr(reinterpret_cast<unsigned long long*>(&w.failm[c >> 6]), 1ULL << (c & 63));
     atomicAdd(w.nfail, 1u);
   };
   int64_t lo = a, hi = b;
-  // (a segment bounded by piece starts alone still counts one failure, so
-  // that the repair pass runs and lists it)
+  // (a segment bounded by piece starts and seams alone still counts one
+  // failure, so that the repair pass runs and lists it)
   if (!is_cut(a) && !is_cut(b)) atomicAdd(w.nfail, 1u);
   if (is_cut(a)) {
     fail(a);
@@ -4185,7 +4567,7 @@ __global__ __launch_bounds__(256) void k_certify(DevTables t, DevWork w,
   const int64_t v = w.vlist[i];
   if (v >= nwords) return;
   if (!all && !word_dirty(w.dirty_cur, v)) return;  // wave-uniform
-  const uint64_t cuts = w.cuts[v] & w.inlong[v] & ~w.starts[v];
+  const uint64_t cuts = w.cuts[v] & w.inlong[v] & ~sure_word(w, v);
   if (!cuts) return;
   // (the long pieces' chain: the first pass runs beside the row merges)
   __builtin_amdgcn_s_setprio(2);
@@ -4252,7 +4634,7 @@ __global__ void k_fail_widen(DevWork w, int64_t nwords, uint32_t width) {
       int64_t wd = v;
       uint64_t m = bit ? (1ULL << bit) - 1 : 0;  // bits below c in its word
       for (;;) {
-        const uint64_t st = w.starts[wd];
+        const uint64_t st = sure_word(w, wd);  // (seams stay)
         uint64_t sb = (st | (w.cuts[wd] & w.inlong[wd])) & m;
         bool done = false;
         while (sb) {
@@ -4279,7 +4661,7 @@ __global__ void k_fail_widen(DevWork w, int64_t nwords, uint32_t width) {
       int64_t wd = v;
       uint64_t m = ~mask_le(bit);  // bits above c in its word
       for (;;) {
-        const uint64_t st = w.starts[wd];
+        const uint64_t st = sure_word(w, wd);  // (seams stay)
         uint64_t sb = (st | (w.cuts[wd] & w.inlong[wd])) & m;
         bool done = false;
         while (sb) {
@@ -4314,26 +4696,50 @@ __global__ void k_fail_widen(DevWork w, int64_t nwords, uint32_t width) {
 // critical path, starved (846 us; 277 us with a quarter of the slots, but
 // the row merge then took 2 ms).
 constexpr uint32_t ROWS_MAX_BLOCKS = 1024;
+hipError_t launch_piece_split(const DevTables& t, const DevWork& w, hipStream_t s,
+                              uint32_t nlong) {
+  hipLaunchKernelGGL(k_piece_split, dim3((nlong + SPLIT_PIECES - 1) / SPLIT_PIECES),
+                     dim3(SPLIT_TPB), 0, s, t, w);
+  return hipGetLastError();
+}
+
+hipError_t launch_bpe_mid(const DevTables& t, const DevWork& w, hipStream_t s,
+                          bool split, uint32_t nmid) {
+  const uint32_t u = nmid / 128 + PACK_XCDS;
+  const uint32_t blocks = split || u > MID_BLOCKS ? MID_BLOCKS : u;
+  hipLaunchKernelGGL(k_bpe_mid, dim3(blocks), dim3(256), 0, s, t, w, split ? 1 : 0,
+                     nmid ? 1 : 0);
+  return hipGetLastError();
+}
+
 hipError_t launch_bpe_rows(const DevTables& t, const DevWork& w, hipStream_t s,
-                           uint32_t nlong, hipEvent_t start, hipEvent_t stop) {
+                           uint32_t nlong, bool split, hipEvent_t start,
+                           hipEvent_t stop) {
   const uint32_t blocks = nlong / 4 + 1 < ROWS_MAX_BLOCKS ? nlong / 4 + 1 : ROWS_MAX_BLOCKS;
   size_t lds = t.unsafe && t.unsafe_words <= ROWS_UNSAFE_LDS
                    ? (size_t)((t.unsafe_words + 3) & ~3u) * 4 : 0;
   if (t.hot) lds += HOT_BYTES;
+  const int sp = split ? 1 : 0;
   if (start || stop)
     hipExtLaunchKernelGGL(k_bpe_rows, dim3(blocks), dim3(256), lds, s, start, stop,
-                          0, t, w);
+                          0, t, w, sp);
   else
-    hipLaunchKernelGGL(k_bpe_rows, dim3(blocks), dim3(256), lds, s, t, w);
+    hipLaunchKernelGGL(k_bpe_rows, dim3(blocks), dim3(256), lds, s, t, w, sp);
   return hipGetLastError();
 }
 
 hipError_t launch_bpe_wide(const DevTables& t, const DevWork& w, hipStream_t s,
-                           hipEvent_t stop, uint32_t nlong) {
+                           hipEvent_t stop, uint32_t nlong, bool split) {
   const uint32_t blocks = nlong / 4 + 1 < 2048 ? nlong / 4 + 1 : 2048;
-  launch_ev(k_bpe_wide, dim3(blocks), dim3(256), s, nullptr, stop, t, w,
-            (const uint32_t*)w.longlist, (const uint32_t*)w.longcount,
-            w.long_cap, 0);
+  const uint32_t* list = w.longlist;
+  const uint32_t* count = w.longcount;
+  uint32_t cap = w.long_cap;
+  if (split) {
+    list = reinterpret_cast<const uint32_t*>(w.parts + part_off(PART_LONG, w.parts_cap));
+    count = w.npart + PART_LONG * CTRL_PART_STRIDE;
+    cap = (uint32_t)part_room(PART_LONG, w.parts_cap);
+  }
+  launch_ev(k_bpe_wide, dim3(blocks), dim3(256), s, nullptr, stop, t, w, list, count, cap, 0);
   return hipGetLastError();
 }
 
@@ -4342,6 +4748,7 @@ hipError_t launch_long_windows(const DevTables& t, const DevWork& w,
   const int64_t nwin = (w.nb + 63) / 64;
   launch_ev(k_win_list, dim3((uint32_t)((nwin + 1 + 255) / 256)), dim3(256), s,
             start, nullptr, w, nwin);
+  hipLaunchKernelGGL(k_long_seams, dim3((uint32_t)((nwin + 4) / 4)), dim3(256), 0, s, t, w);
   launch_ev(k_long_windows, dim3((uint32_t)((nwin + 4) / 4)), dim3(256), s, nullptr,
             stop, t, w, nwin);
   return hipGetLastError();

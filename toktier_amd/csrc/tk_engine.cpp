@@ -204,6 +204,82 @@ bool place_pairs(const PairEntries& ent, size_t n, uint32_t bits,
   }
 }
 
+// The strings that a symbol can spell: the bytes of every rule's product
+// (from the rules alone: product = left + right) and, for tables with a
+// whole-piece rule, the vocabulary entries. False when they are not plain
+// (a byte without an id, an id with two spellings, entries out of the blob):
+// the engine then looks for no seams. A rule whose sides no byte sequence
+// reaches never runs and spells nothing.
+bool symbol_strings(const uint64_t* keys, const uint64_t* vals, uint64_t count,
+                    const int32_t* byte_id, std::vector<std::string>& out) {
+  constexpr size_t MAX_LEN = 4096;  // (far above any token; bounds the memory)
+  std::vector<std::string> of;      // by id
+  auto put = [&](uint64_t id, std::string s) {
+    if (id >= of.size()) of.resize(id + 1);
+    if (of[id].empty()) of[id] = std::move(s);
+    else if (of[id] != s) return false;
+    return true;
+  };
+  for (int b = 0; b < 256; ++b)
+    if (byte_id[b] < 0 || !put((uint64_t)byte_id[b], std::string(1, (char)b))) return false;
+  struct Rule { uint64_t rank, l, r, id; };
+  std::vector<Rule> todo;
+  for (uint64_t i = 0; i < count; ++i)
+    if (keys[i] != ~0ULL)
+      todo.push_back({vals[i] >> 32, keys[i] >> 32, keys[i] & 0xFFFFFFFFULL,
+                      vals[i] & 0xFFFFFFFFULL});
+  std::sort(todo.begin(), todo.end(),
+            [](const Rule& a, const Rule& b) { return a.rank < b.rank; });
+  // (in rank order nearly every rule's sides are known by its turn)
+  for (size_t left = todo.size() + 1; todo.size() < left && !todo.empty();) {
+    left = todo.size();
+    std::vector<Rule> later;
+    for (const Rule& u : todo) {
+      if (u.l >= of.size() || u.r >= of.size() || of[u.l].empty() || of[u.r].empty()) {
+        later.push_back(u);
+        continue;
+      }
+      std::string s = of[u.l] + of[u.r];
+      if (s.size() > MAX_LEN || !put(u.id, s)) return false;
+      out.push_back(std::move(s));
+    }
+    todo.swap(later);
+  }
+  return true;
+}
+
+// The seam tables (tk_device.h) of those strings: every inner position of
+// every string, as its byte pair's key type and its key. The bitmap has at
+// least 16 bits per key, up to 2^24 (2 MB).
+struct SeamTables {
+  std::vector<uint16_t> mask;
+  std::vector<uint32_t> bits;
+  uint32_t shift = 0;
+};
+void build_seams(const std::vector<std::string>& strings, SeamTables& t) {
+  size_t keys = 0;
+  for (const std::string& s : strings) keys += s.size();
+  uint32_t lg = 16;
+  while (lg < 24 && ((size_t)1 << lg) < 8 * keys) ++lg;  // (half the keys repeat)
+  t.mask.assign(65536, 0);
+  t.bits.assign((size_t)1 << (lg - 5), 0);
+  t.shift = 32 - lg;
+  for (const std::string& s : strings) {
+    const uint8_t* p = reinterpret_cast<const uint8_t*>(s.data());
+    for (size_t i = 1; i < s.size(); ++i) {
+      const int A = (int)std::min<size_t>(i, tk::SEAM_CTX);
+      const int B = (int)std::min<size_t>(s.size() - i, tk::SEAM_CTX);
+      uint32_t left = 0, right = 0;
+      for (int k = 0; k < A; ++k) left |= (uint32_t)p[i - 1 - k] << (8 * k);
+      for (int k = 0; k < B; ++k) right |= (uint32_t)p[i + k] << (8 * k);
+      const uint32_t type = (uint32_t)((A - 1) * tk::SEAM_CTX + (B - 1));
+      t.mask[(size_t)p[i - 1] << 8 | p[i]] |= (uint16_t)(1u << type);
+      const uint32_t h = tk::seam_hash(left, right, type) >> t.shift;
+      t.bits[h >> 5] |= 1u << (h & 31);
+    }
+  }
+}
+
 // One request's device workspace: every per-call buffer, carved out of one
 // region -- the engine's own allocation, or, for
 // tk_engine_encode_device_noalloc, the library's static scratch array.
@@ -215,10 +291,11 @@ struct Workspace {
   size_t cap = 0;  // input bytes the workspace holds
   uint8_t* text = nullptr;
   uint64_t *starts = nullptr, *docmask = nullptr, *heap = nullptr;
-  uint64_t *cstat = nullptr, *inlong = nullptr, *cuts = nullptr;
+  uint64_t *cstat = nullptr, *inlong = nullptr, *cuts = nullptr, *sure = nullptr;
   uint64_t *failm = nullptr, *hfirst = nullptr, *hlast = nullptr;
   uint64_t *dirty_cur = nullptr, *dirty_next = nullptr;
   uint64_t *lits = nullptr, *litb = nullptr, *docmask_lit = nullptr;
+  uint2* parts = nullptr;  // parts of the queued pieces, by class
   uint64_t* nrun = nullptr;  // per k_pretok tile: the digit run, then two
                              // automaton words (o200k)
   uint32_t *tok = nullptr, *longlist = nullptr, *ctrl = nullptr;
@@ -234,7 +311,7 @@ struct Workspace {
 
 // Lays a workspace for `cap` input bytes out at `base` (each buffer
 // 256-byte aligned) and returns the bytes it spans; base == nullptr only
-// sizes it. About 70 bytes per input byte.
+// sizes it. About 80 bytes per input byte.
 size_t carve(Workspace& w, uint8_t* base, size_t cap) {
   size_t at = 0;
   auto take = [&](auto*& p, size_t count) {
@@ -265,6 +342,7 @@ size_t carve(Workspace& w, uint8_t* base, size_t cap) {
   take(w.ctrl, 2 * tk::CTRL_WORDS);  // two control slots
   take(w.inlong, words);
   take(w.cuts, words);
+  take(w.sure, words);
   take(w.failm, words);
   take(w.hfirst, cap);
   take(w.hlast, cap);
@@ -281,6 +359,7 @@ size_t carve(Workspace& w, uint8_t* base, size_t cap) {
   take(w.lits, words);
   take(w.litb, words);
   take(w.docmask_lit, words);
+  take(w.parts, tk::part_off(tk::PART_CLASSES, cap));
   take(w.nrun, 3 * (size_t)tiles);
   w.cap = cap;
   w.tiles = (size_t)tiles;
@@ -303,6 +382,8 @@ struct tk_engine {
   DevBuf<ulonglong2> pairs, vocab;
   DevBuf<uint64_t> bytepair, ctab, hot;
   uint32_t hot_k = 0;  // rules of rank below it are in `hot`
+  DevBuf<uint16_t> seam_mask;
+  DevBuf<uint32_t> seam_bits;
   DevBuf<int32_t> byte_id;
   std::vector<uint8_t> host_nfc;
   tk::DevTables t{};
@@ -463,6 +544,7 @@ tk::DevWork make_work(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   w.out_cap = (uint32_t)std::min<size_t>(out_cap, 0xFFFFFFFFu);
   w.inlong = ws.inlong;
   w.cuts = ws.cuts;
+  w.sure = ws.sure;
   w.failm = ws.failm;
   w.hfirst = ws.hfirst;
   w.hlast = ws.hlast;
@@ -483,6 +565,9 @@ tk::DevWork make_work(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   w.nbig = ctrl + tk::CTRL_BIG;
   w.prepdone = ctrl + tk::CTRL_PREP;
   w.nwide = ctrl + tk::CTRL_WIDE;
+  w.parts = ws.parts;
+  w.parts_cap = ws.cap;
+  w.npart = ctrl + tk::CTRL_PART;
   w.nrows = ctrl + tk::CTRL_ROWS;
   w.rowq = ctrl + tk::CTRL_ROWQ;
   w.vlist = ws.vlist;
@@ -648,9 +733,16 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   const uint32_t big = cut ? e->gate[tk::GATE_BIG] : 0;
   e->last_nlong = nlong;
   e->last_big = e->gate[tk::GATE_BIG];
-  // (pieces of 65..128 bytes are k_bpe_rows' too past PACK_ROWS_MAX)
-  const bool rows = nrows > 0 || nlong > (uint32_t)tk::PACK_ROWS_MAX;
-  const bool side2 = rows || nwide > 0 ||
+  // (past PACK_ROWS_MAX the queued pieces are cut at their seams and merged
+  // part by part, or whole by k_bpe_rows; past PACK_MID_MAX the listed ones
+  // of 33..64 bytes are k_bpe_mid's)
+  const bool many = nlong > (uint32_t)tk::PACK_ROWS_MAX;
+  const bool split = many && tk::mid_table(e->t);
+  const uint32_t nmid = tk::mid_table(e->t) && e->gate[tk::GATE_NMID] > (uint32_t)tk::PACK_MID_MAX
+                            ? e->gate[tk::GATE_NMID] : 0;
+  // (a part over 128 bytes is of a piece over 128 bytes)
+  const bool rows = nrows > 0 || (split ? nwide > 0 : many);
+  const bool side2 = split || nmid || rows || nwide > 0 ||
                      (!cut && e->gate[tk::GATE_BIG] > 0);
   {
     // two independent jobs on two side streams: the cut / segment / certify
@@ -663,13 +755,18 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
       HIP_TRY(tk::launch_long_windows(e->t, w, s3, ks(TK_KERNEL_LONG_WINDOWS),
                                       ke(TK_KERNEL_LONG_WINDOWS)));
       launched[TK_KERNEL_LONG_WINDOWS] = true;
-      // the row merges next (their launch is not held behind the chain's
-      // twenty-odd launches on the host)
-      if (rows) {
-        HIP_TRY(tk::launch_bpe_rows(e->t, w, s2, nlong, ks(TK_KERNEL_BPE_ROWS),
-                                    ke(TK_KERNEL_BPE_ROWS)));
-        launched[TK_KERNEL_BPE_ROWS] = true;
-      }
+    }
+    // the merges of the queued pieces next (after the chain's first kernel,
+    // so that one is dispatched first; their launches are not held behind
+    // the chain's twenty-odd launches on the host)
+    if (split) HIP_TRY(tk::launch_piece_split(e->t, w, s2, nlong));
+    if (split || nmid) HIP_TRY(tk::launch_bpe_mid(e->t, w, s2, split, nmid));
+    if (rows) {
+      HIP_TRY(tk::launch_bpe_rows(e->t, w, s2, nlong, split, ks(TK_KERNEL_BPE_ROWS),
+                                  ke(TK_KERNEL_BPE_ROWS)));
+      launched[TK_KERNEL_BPE_ROWS] = true;
+    }
+    if (big) {
       HIP_TRY(tk::launch_long_segments(e->t, w, s3));
       HIP_TRY(tk::launch_seg_lists(e->t, w, s3));
       HIP_TRY(tk::launch_certify(e->t, w, 1, s3));
@@ -682,13 +779,7 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
       HIP_TRY(hipEventRecord(e->ev_join3, s3));
       HIP_TRY(hipStreamWaitEvent(s, e->ev_join3, 0));
     }
-    // (after the chain's first kernel, so that one is dispatched first)
-    if (rows && !big) {
-      HIP_TRY(tk::launch_bpe_rows(e->t, w, s2, nlong, ks(TK_KERNEL_BPE_ROWS),
-                                  ke(TK_KERNEL_BPE_ROWS)));
-      launched[TK_KERNEL_BPE_ROWS] = true;
-    }
-    if (nwide > 0) HIP_TRY(tk::launch_bpe_wide(e->t, w, s2, nullptr, nlong));
+    if (nwide > 0) HIP_TRY(tk::launch_bpe_wide(e->t, w, s2, nullptr, nlong, split));
     // (a table that drops bytes merges its pieces over WIDE_MAX bytes
     // whole, a workgroup each, after the wide merges)
     if (!cut && e->gate[tk::GATE_BIG] > 0)
@@ -1176,6 +1267,26 @@ int tk_engine_open(const tk_config* cfg, const uint8_t* class_table,
         if ((rc = up(e->hot, ht.data(), ht.size())) != TK_OK) return bail(rc);
         e->hot_k = hk;
       }
+    }
+  }
+  e->t.seam_mask = nullptr;
+  {
+    std::vector<std::string> strings;
+    bool plain = symbol_strings(pair_keys, pair_vals, n_pairs, byte_id, strings);
+    for (uint64_t i = 0; plain && cfg->ignore_merges && i < cfg->vocab_count; ++i) {
+      if (vocab_keys[i] == ~0ULL) continue;
+      const uint64_t off = vocab_vals[i] >> 30, len = (vocab_vals[i] >> 20) & 0x3FF;
+      plain = off <= vocab_blob_len && len <= vocab_blob_len - off;
+      if (plain) strings.emplace_back(reinterpret_cast<const char*>(vocab_blob) + off, len);
+    }
+    if (plain) {
+      SeamTables st;
+      build_seams(strings, st);
+      if ((rc = up(e->seam_mask, st.mask.data(), st.mask.size())) != TK_OK) return bail(rc);
+      if ((rc = up(e->seam_bits, st.bits.data(), st.bits.size())) != TK_OK) return bail(rc);
+      e->t.seam_mask = e->seam_mask.p;
+      e->t.seam_bits = e->seam_bits.p;
+      e->t.seam_shift = st.shift;
     }
   }
   e->t.unsafe = nullptr;
