@@ -628,23 +628,28 @@ int read_ctrl_words(const uint32_t* ctrl, hipStream_t s, uint32_t* h) {
   return TK_OK;
 }
 
-// Wait until k_bpe_pack of call `seq` has written the gate words (a
-// spin on host memory). A device fault would stop the writer, so after a
-// generous bound the stream is synchronized to surface its error.
-int wait_gate(tk_engine* e, uint32_t seq, hipStream_t s) {
+// Spin on a gate word until the device has written call `seq` there; false
+// after a generous bound (a device fault would stop the writer: the caller
+// then synchronizes the stream, which surfaces its error).
+bool wait_word(tk_engine* e, int word, uint32_t seq) {
   const auto t0 = std::chrono::steady_clock::now();
   for (uint64_t spin = 0;; ++spin) {
-    if (e->gate[tk::GATE_SEQ] == seq) {
+    if (e->gate[word] == seq) {
       std::atomic_thread_fence(std::memory_order_acquire);
-      return TK_OK;
+      return true;
     }
     if ((spin & 1023) == 1023 &&
-        std::chrono::steady_clock::now() - t0 > std::chrono::seconds(10)) {
-      HIP_TRY(hipStreamSynchronize(s));
-      if (e->gate[tk::GATE_SEQ] == seq) return TK_OK;
-      return fail(TK_E_INTERNAL, "gate words were not written");
-    }
+        std::chrono::steady_clock::now() - t0 > std::chrono::seconds(10))
+      return false;
   }
+}
+
+// Wait until k_bpe_pack of call `seq` has written the gate words.
+int wait_gate(tk_engine* e, uint32_t seq, hipStream_t s) {
+  if (wait_word(e, tk::GATE_SEQ, seq)) return TK_OK;
+  HIP_TRY(hipStreamSynchronize(s));
+  if (e->gate[tk::GATE_SEQ] == seq) return TK_OK;
+  return fail(TK_E_INTERNAL, "gate words were not written");
 }
 
 float elapsed_us(hipEvent_t a, hipEvent_t b) {
@@ -677,13 +682,14 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
                  hipStream_t s, uint32_t* out, size_t out_cap,
                  uint32_t* status, uint32_t* total,
                  const tk::DevAdded* docs = nullptr,
-                 const RowsOut* rows_out = nullptr) {
+                 const RowsOut* rows_out = nullptr, const uint8_t* src = nullptr) {
   ++e->seq;
   const bool literals = docs != nullptr;
   const uint64_t* host_dm = d_docmask;
   if (literals) d_docmask = ws.docmask_lit;
-  const tk::DevWork w = make_work(e, ws, d_text, nb, d_docmask, check_nfc,
-                                  out, out_cap, literals);
+  tk::DevWork w = make_work(e, ws, d_text, nb, d_docmask, check_nfc,
+                            out, out_cap, literals);
+  w.src = src;  // (host-mapped; k_added, which then runs, brings it to d_text)
   uint32_t* ctrl = ws.ctrl + ws.slot * tk::CTRL_WORDS;
   hipEvent_t* ev = e->ev;
   // Timing mode 1: every kernel of TK_KERNEL_* takes a start / stop event
@@ -795,14 +801,22 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   // the compaction reports the failed cuts left after the last queued pass
   tk::DevWork wc = w;
   if (big) wc.nfail = fail_count(ctrl, DEV_REPAIRS);
+  // a small request with nothing behind its compaction: the outcome words end
+  // the call, 3..4 us before the stream counts as done. Not one whose text was
+  // sent by a copy command: the next call's command then waits for this
+  // kernel's end in the queue (a 64 KiB host call 86 -> 90 us)
+  const bool spin = !rows_out && e->timing == 0 && (src || d_text != ws.text) &&
+                    nb <= (size_t)(tk::DONE_BLOCKS * tk::COMPACT_BLOCK);
+  if (spin) wc.ndone = ctrl + tk::CTRL_DONE;
   HIP_TRY(tk::launch_compact(wc, s, ++ws.ctag, ks(TK_KERNEL_COMPACT),
                              ke(TK_KERNEL_COMPACT)));
   launched[TK_KERNEL_COMPACT] = true;
   if (rows_out)
     HIP_TRY(tk::launch_doc_offsets(w, rows_out->offs, rows_out->n, rows_out->rows, s));
+  wc.ndone = nullptr;
   // k_compact's last block has left the outcome in the gate words: no
   // read-back copy
-  HIP_TRY(hipStreamSynchronize(s));
+  if (!spin || !wait_word(e, tk::GATE_DONE, w.seq)) HIP_TRY(hipStreamSynchronize(s));
   uint32_t* h = e->host_ctrl;
   if (e->gate[tk::GATE_DONE] != w.seq)
     return fail(TK_E_INTERNAL, "outcome words were not written");
@@ -872,6 +886,11 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
 
 // ---- host <-> device through the pinned staging
 constexpr size_t STAGE_SMALL = (size_t)256 << 10;  // one copy, this thread
+// Up to here k_added reads a host call's bytes from the pinned staging: 64 KiB
+// of ascii 86 -> 77 us, 400,000 bytes 108 -> 101, 512 KiB 115 -> 111; 1 MiB
+// 147 -> 170 (each block reads its margins over PCIe again, and the bytes
+// come only as fast as the blocks in flight ask for them).
+constexpr size_t MAP_SMALL = (size_t)512 << 10;
 constexpr size_t STAGE_CHUNK = (size_t)64 << 10;   // one claim of the copy threads
 
 tk::CopyPool* copy_pool(tk_engine* e) {
@@ -929,8 +948,8 @@ void host_copy(tk_engine* e, uint8_t* dst, const uint8_t* src, size_t n) {
 
 // n request bytes at src (host) into d_dst (device) on stream s: page-locked
 // bytes in one transfer; pageable ones copied into the pinned staging
-// first, then one transfer (the staging is free again once the call has
-// synchronized, as every host entry does before it returns).
+// first, then one transfer (the staging is free again once the call's
+// kernels are done with it, which every host entry waits for).
 int stage_in(tk_engine* e, uint8_t* d_dst, const uint8_t* src, size_t n,
              hipStream_t s) {
   if (pinned_range(src, n)) {
@@ -940,6 +959,20 @@ int stage_in(tk_engine* e, uint8_t* d_dst, const uint8_t* src, size_t n,
   HIP_TRY(e->pin_in.ensure(std::max(n, e->ws.cap) + 64));
   host_copy(e, e->pin_in.p, src, n);
   HIP_TRY(hipMemcpyAsync(d_dst, e->pin_in.p, n, hipMemcpyHostToDevice, s));
+  return TK_OK;
+}
+
+// The same for a request that k_added reads first: up to MAP_SMALL pageable
+// bytes stay in the pinned staging, and *mapped is the device's address of
+// them (k_added brings them over: no copy command, no wait for one); *mapped
+// stays nullptr when they were sent.
+int stage_small(tk_engine* e, uint8_t* d_dst, const uint8_t* src, size_t n,
+                bool added, hipStream_t s, const uint8_t** mapped) {
+  *mapped = nullptr;
+  if (!added || n > MAP_SMALL || pinned_range(src, n)) return stage_in(e, d_dst, src, n, s);
+  HIP_TRY(e->pin_in.ensure(std::max(n, e->ws.cap) + 64));
+  host_copy(e, e->pin_in.p, src, n);
+  *mapped = e->pin_in.dev;
   return TK_OK;
 }
 
@@ -1679,14 +1712,17 @@ int tk_engine_encode_seed_host(tk_engine* e, const uint8_t* text, size_t nbytes,
   int rc = ensure_workspace(e, nbytes, 0);
   if (rc != TK_OK) return rc;
   hipStream_t s = e->stream;
-  if ((rc = stage_in(e, e->ws.text, text, nbytes, s)) != TK_OK) return rc;
+  tk::DevAdded docs;
+  const tk::DevAdded* const dp = doc_pass(e, flags, &docs);
+  const uint8_t* mapped;
+  if ((rc = stage_small(e, e->ws.text, text, nbytes, dp != nullptr, s, &mapped)) != TK_OK)
+    return rc;
   HostOut o;
   if ((rc = host_out(e, ids, ids_cap, &o)) != TK_OK) return rc;
   const bool check = e->t.needs_nfc && !(flags & TK_FLAG_NORMALIZED);
   uint32_t st, total;
-  tk::DevAdded docs;
   rc = run_pipeline(e, e->ws, e->ws.text, nbytes, nullptr, check, s, o.dev,
-                    o.cap, &st, &total, doc_pass(e, flags, &docs));
+                    o.cap, &st, &total, dp, nullptr, mapped);
   if (rc != TK_OK) return rc;
   if (st & tk::ST_UTF8) return fail(TK_E_UTF8, "input is not valid UTF-8");
   if (st & tk::ST_NFC) return fail(TK_E_NEEDS_NFC, "NFC quick check failed");
@@ -1732,15 +1768,18 @@ int tk_engine_encode(tk_engine* e, const uint8_t* text, size_t nbytes,
   hipStream_t s = e->stream;
   using clk = std::chrono::steady_clock;
   const auto h0 = clk::now();
-  if ((rc = stage_in(e, e->ws.text, text, nbytes, s)) != TK_OK) return rc;
+  tk::DevAdded docs;
+  const tk::DevAdded* const dp = doc_pass(e, flags, &docs);
+  const uint8_t* mapped;
+  if ((rc = stage_small(e, e->ws.text, text, nbytes, dp != nullptr, s, &mapped)) != TK_OK)
+    return rc;
   HostOut o;
   if ((rc = host_out(e, ids, ids_cap, &o)) != TK_OK) return rc;
   const auto h1 = clk::now();
   const bool check = e->t.needs_nfc && !(flags & TK_FLAG_NORMALIZED);
   uint32_t st, total;
-  tk::DevAdded docs;
   rc = run_pipeline(e, e->ws, e->ws.text, nbytes, nullptr, check, s, o.dev,
-                    o.cap, &st, &total, doc_pass(e, flags, &docs));
+                    o.cap, &st, &total, dp, nullptr, mapped);
   const auto h2 = clk::now();
   if (rc != TK_OK) return rc;
   if (st & tk::ST_UTF8) return fail(TK_E_UTF8, "input is not valid UTF-8");

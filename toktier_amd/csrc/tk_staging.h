@@ -23,7 +23,8 @@
 namespace tk {
 
 // Pinned host memory (hipHostMalloc), grown on demand.
-// `dev` is its address in the device's view, for kernels that write it.
+// `dev` is its address in the device's view, for kernels that read or write
+// it (coherent: a kernel never reads a line kept from an earlier call).
 struct PinnedBuf {
   uint8_t* p = nullptr;
   uint8_t* dev = nullptr;
@@ -39,7 +40,7 @@ struct PinnedBuf {
     if (bytes <= n) return hipSuccess;
     reset();
     void* q = nullptr;
-    hipError_t e = hipHostMalloc(&q, bytes, hipHostMallocDefault);
+    hipError_t e = hipHostMalloc(&q, bytes, hipHostMallocMapped | hipHostMallocCoherent);
     if (e != hipSuccess) return e;
     void* d = nullptr;
     e = hipHostGetDevicePointer(&d, q, 0);
