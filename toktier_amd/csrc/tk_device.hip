@@ -4151,52 +4151,50 @@ __device__ __forceinline__ uint64_t sure_word(const DevWork& w, int64_t wd) {
 }
 
 __device__ __forceinline__ void long_window(const DevTables& t, const DevWork& w,
-                                            int64_t v, int64_t nwin) {
+                                            int64_t v, int phase) {
   const int lane = threadIdx.x & 63;
   auto seg = [&](int64_t wd) { return wd < 0 ? ~0ULL : sure_word(w, wd); };
   uint16_t* cut16 = reinterpret_cast<uint16_t*>(w.cuts);
   const uint16_t* sure16 = reinterpret_cast<const uint16_t*>(w.sure);
-  for (int phase = (v == nwin ? 1 : 0); phase < 2; ++phase) {
-    const uint64_t L = inlong_window(w, v, phase);
-    if (L == 0) continue;  // wave-uniform
-    const int64_t base = phase == 0 ? v * 64 : v * 64 - 32;
-    // the boundaries in the window (S) and in the 64 bytes either side
-    const uint64_t b0 = seg(v - 1), b1 = seg(v), b2 = seg(v + 1);
-    uint64_t S, below, above;
+  const uint64_t L = inlong_window(w, v, phase);
+  if (L == 0) return;  // wave-uniform
+  const int64_t base = phase == 0 ? v * 64 : v * 64 - 32;
+  // the boundaries in the window (S) and in the 64 bytes either side
+  const uint64_t b0 = seg(v - 1), b1 = seg(v), b2 = seg(v + 1);
+  uint64_t S, below, above;
+  if (phase == 0) {
+    S = b1;
+    below = b0;
+    above = b2;
+  } else {
+    S = (b0 >> 32) | (b1 << 32);
+    below = (seg(v - 2) >> 32) | (b0 << 32);
+    above = (b1 >> 32) | (b2 << 32);
+  }
+  // the lane's stretch between two of them: over 64 bytes?
+  const uint64_t sle = S & mask_le(lane), sgt = S & ~mask_le(lane);
+  const int back = sle ? lane - (63 - __builtin_clzll(sle))
+                 : below ? lane + 1 + __builtin_clzll(below) : 128;
+  const int fwd = sgt ? __builtin_ctzll(sgt) - lane
+                : above ? 64 - lane + __builtin_ctzll(above) : 128;
+  const uint64_t far = __ballot(back + fwd > 64 && ((L >> lane) & 1)) & 0x0000FFFFFFFF0000ULL;
+  uint64_t live = 0;
+  if (far) {  // wave-uniform
+    S |= 1;  // the window start cuts whatever runs into it
+    const uint64_t le = S & mask_le(lane);
+    const int ps = 63 - __builtin_clzll(le);
+    const uint64_t gt = S & ~mask_le(lane);
+    const int pe = gt ? __builtin_ctzll(gt) : 64;
+    const bool elig = (L >> lane) & 1;
+    live = wave_bpe<false, false, false>(t, w, base, base + lane, lane, elig, ps, pe) & far;
+  }
+  if (lane == 0) {
     if (phase == 0) {
-      S = b1;
-      below = b0;
-      above = b2;
+      cut16[4 * v + 1] = (uint16_t)(live >> 16) | sure16[4 * v + 1];
+      cut16[4 * v + 2] = (uint16_t)(live >> 32) | sure16[4 * v + 2];
     } else {
-      S = (b0 >> 32) | (b1 << 32);
-      below = (seg(v - 2) >> 32) | (b0 << 32);
-      above = (b1 >> 32) | (b2 << 32);
-    }
-    // the lane's stretch between two of them: over 64 bytes?
-    const uint64_t sle = S & mask_le(lane), sgt = S & ~mask_le(lane);
-    const int back = sle ? lane - (63 - __builtin_clzll(sle))
-                   : below ? lane + 1 + __builtin_clzll(below) : 128;
-    const int fwd = sgt ? __builtin_ctzll(sgt) - lane
-                  : above ? 64 - lane + __builtin_ctzll(above) : 128;
-    const uint64_t far = __ballot(back + fwd > 64 && ((L >> lane) & 1)) & 0x0000FFFFFFFF0000ULL;
-    uint64_t live = 0;
-    if (far) {  // wave-uniform
-      S |= 1;  // the window start cuts whatever runs into it
-      const uint64_t le = S & mask_le(lane);
-      const int ps = 63 - __builtin_clzll(le);
-      const uint64_t gt = S & ~mask_le(lane);
-      const int pe = gt ? __builtin_ctzll(gt) : 64;
-      const bool elig = (L >> lane) & 1;
-      live = wave_bpe<false, false, false>(t, w, base, base + lane, lane, elig, ps, pe) & far;
-    }
-    if (lane == 0) {
-      if (phase == 0) {
-        cut16[4 * v + 1] = (uint16_t)(live >> 16) | sure16[4 * v + 1];
-        cut16[4 * v + 2] = (uint16_t)(live >> 32) | sure16[4 * v + 2];
-      } else {
-        if (v > 0) cut16[4 * (v - 1) + 3] = (uint16_t)(live >> 16) | sure16[4 * (v - 1) + 3];
-        cut16[4 * v] = (uint16_t)(live >> 32) | sure16[4 * v];
-      }
+      if (v > 0) cut16[4 * (v - 1) + 3] = (uint16_t)(live >> 16) | sure16[4 * (v - 1) + 3];
+      cut16[4 * v] = (uint16_t)(live >> 32) | sure16[4 * v];
     }
   }
 }
@@ -4204,17 +4202,23 @@ __device__ __forceinline__ void long_window(const DevTables& t, const DevWork& w
 // Cut selection: BPE of the long-piece bytes of every window that a stretch
 // of over 64 bytes between seams (or piece ends) reaches into, window edges
 // taken as cuts; the token starts of such stretches in the window's central
-// 32 bytes become candidate cuts, beside the seams. Aligned window v owns bits 16..47 of word v, shifted
-// window v owns bits 48..63 of word v-1 and 0..15 of word v. Wave i takes
-// listed window i.
+// 32 bytes become candidate cuts, beside the seams. Aligned window v owns bits
+// 16..47 of word v, shifted window v owns bits 48..63 of word v-1 and 0..15 of
+// word v. Waves 2i and 2i + 1 take the two phases of listed window i: they
+// write different quarters of the words, and latency bounds the kernel, so a
+// wave that merged both made its chain twice as long. 1,048,577 chars of CJK
+// text with two 65,536-letter runs (DeepSeek): k_long_windows 85 -> 61 us,
+// k_long_segments, split alike, 69 -> 60, the call 575 -> 547; with ten runs
+// in 4,194,304 chars (Qwen3) 194 -> 167 and 198 -> 194, 1,060 -> 1,056.
 __global__ __launch_bounds__(256) void k_long_windows(DevTables t, DevWork w,
                                                       int64_t nwin) {
-  const uint32_t i = blockIdx.x * 4 + wave_id();
+  const uint32_t k = blockIdx.x * 4 + wave_id(), i = k >> 1;
   if (i >= *w.vcount) return;
   // the long pieces' chain (windows, segments, certification, repairs)
   // sets the end of a request that has any: issue priority
   __builtin_amdgcn_s_setprio(2);
-  long_window(t, w, w.vlist[i], nwin);
+  const int64_t v = w.vlist[i];
+  if ((k & 1) || v < nwin) long_window(t, w, v, (int)(k & 1));
 }
 
 __device__ __forceinline__ uint64_t seg_word(const DevWork& w, int64_t wd) {
@@ -4303,18 +4307,18 @@ __device__ __forceinline__ void segment_window(const DevTables& t, const DevWork
 }
 
 // Segment pass over the long-piece bytes (64-byte grid windows, aligned and
-// shifted by 32, with histories), wave i over listed window i. Segments
+// shifted by 32, with histories), waves 2i and 2i + 1 over the two phases of
+// listed window i (they hold different segments). Segments
 // that fit no grid window go to seglist. (The
 // repair passes redo only the windows of dirty words: k_seg_scan,
 // k_repair_merge.)
 __global__ __launch_bounds__(256) void k_long_segments(DevTables t, DevWork w,
                                                        int64_t nwin) {
-  const uint32_t i = blockIdx.x * 4 + wave_id();
+  const uint32_t k = blockIdx.x * 4 + wave_id(), i = k >> 1;
   if (i >= *w.vcount || !pass_live(w)) return;
   __builtin_amdgcn_s_setprio(2);  // (the long pieces' chain: k_long_windows)
   const int64_t v = w.vlist[i];
-  for (int phase = (v == nwin ? 1 : 0); phase < 2; ++phase)
-    segment_window(t, w, v, phase, true);
+  if ((k & 1) || v < nwin) segment_window(t, w, v, (int)(k & 1), true);
 }
 
 // A repair pass's work list, one thread per text word d: when d is dirty,
@@ -4390,8 +4394,8 @@ __global__ __launch_bounds__(256) void k_repair_merge(DevTables t, DevWork w,
   const int wv = wave_id();
   const uint32_t waves = gridDim.x * 4;
   // (the long pieces' chain, as k_bpe_wide's segments with histories)
-  if (blockIdx.x * 4 + wv < ns + nw) __builtin_amdgcn_s_setprio(3);
-  for (uint32_t k = blockIdx.x * 4 + wv; k < ns + nw; k += waves) {
+  if (blockIdx.x * 4 + wv < ns + 2 * nw) __builtin_amdgcn_s_setprio(3);
+  for (uint32_t k = blockIdx.x * 4 + wv; k < ns + 2 * nw; k += waves) {
     if (k < ns) {
       const uint32_t a = w.seglist[2 * k], b = w.seglist[2 * k + 1];
       const int len = (int)(b - a);
@@ -4406,10 +4410,10 @@ __global__ __launch_bounds__(256) void k_repair_merge(DevTables t, DevWork w,
       else if (len <= WIDE_MAX)
         wave_bpe_wide(t, w, a, len, false, true, lds[wv]);
     } else {
-      const uint32_t it = w.wlist[k - ns];
-      const int64_t v = (int64_t)(it >> 1);
-      if (it & 1) segment_window(t, w, v, 0, false);
-      segment_window(t, w, v, 1, false);
+      // (the windows' phase 1 first, then the phase 0 of those that have it)
+      const uint32_t at = k - ns, it = w.wlist[at < nw ? at : at - nw];
+      if (at < nw || (it & 1))
+        segment_window(t, w, (int64_t)(it >> 1), at < nw ? 1 : 0, false);
     }
   }
 }
@@ -4749,14 +4753,14 @@ hipError_t launch_long_windows(const DevTables& t, const DevWork& w,
   launch_ev(k_win_list, dim3((uint32_t)((nwin + 1 + 255) / 256)), dim3(256), s,
             start, nullptr, w, nwin);
   hipLaunchKernelGGL(k_long_seams, dim3((uint32_t)((nwin + 4) / 4)), dim3(256), 0, s, t, w);
-  launch_ev(k_long_windows, dim3((uint32_t)((nwin + 4) / 4)), dim3(256), s, nullptr,
+  launch_ev(k_long_windows, dim3((uint32_t)((nwin + 2) / 2)), dim3(256), s, nullptr,
             stop, t, w, nwin);
   return hipGetLastError();
 }
 
 hipError_t launch_long_segments(const DevTables& t, const DevWork& w, hipStream_t s) {
   const int64_t nwin = (w.nb + 63) / 64;
-  hipLaunchKernelGGL(k_long_segments, dim3((uint32_t)((nwin + 4) / 4)), dim3(256), 0,
+  hipLaunchKernelGGL(k_long_segments, dim3((uint32_t)((nwin + 2) / 2)), dim3(256), 0,
                      s, t, w, nwin);
   return hipGetLastError();
 }
