@@ -5126,22 +5126,44 @@ hipError_t launch_seed(const DevWork& w, const uint8_t* text, int64_t nb,
 
 // row d starts at the number of tokens whose first byte lies before
 // doc_offsets[d]: the compaction's prefix at its block plus the token slots
-// of the block before it, counted by one wave (lanes strided, then a wave
-// sum)
-__global__ __launch_bounds__(256) void k_doc_offsets(DevWork w,
-                                                     const uint64_t* doc_offsets,
-                                                     uint32_t n, uint64_t* rows) {
-  const uint32_t d = blockIdx.x * 4 + wave_id();
-  if (d > n) return;  // wave-uniform
-  const int lane = threadIdx.x & 63;
+// of the block before it, counted by a workgroup with all of its loads in
+// flight at once. (A wave a row, a 4-byte slot a lane and step, was a chain of
+// up to 128 loads: 38 us for 256 rows as for 1,500, now 6.9 for 1,500. The
+// calls: 1,500 documents of 700,000 chars 480 -> 450 us, 256 of 4,300,000
+// 477 -> 445.)
+__global__ __launch_bounds__(COMPACT_TPB) void k_doc_offsets(DevWork w,
+                                                             const uint64_t* doc_offsets,
+                                                             uint64_t* rows) {
+  constexpr int STEPS = COMPACT_PER_THREAD / 4, WAVES = COMPACT_TPB / 64;
+  __shared__ uint32_t part[WAVES];
+  const uint32_t d = blockIdx.x;
+  const int tid = threadIdx.x;
   int64_t p = (int64_t)doc_offsets[d];
   if (p > w.nb) p = w.nb;
-  const int64_t blk = p / COMPACT_BLOCK;
+  const int64_t blk = p / COMPACT_BLOCK, first = blk * COMPACT_BLOCK;
+  const int n = (int)(p - first);  // slots to count, below COMPACT_BLOCK
+  // (16-byte loads: the slots are allocated in whole 16-byte groups)
+  uint4 v[STEPS];
+#pragma unroll
+  for (int j = 0; j < STEPS; ++j) {
+    const int q = 4 * (tid + j * COMPACT_TPB);
+    v[j] = make_uint4(INVALID_ID, INVALID_ID, INVALID_ID, INVALID_ID);
+    if (q < n) v[j] = *reinterpret_cast<const uint4*>(w.tok + first + q);
+  }
   uint32_t c = 0;
-  for (int64_t q = blk * COMPACT_BLOCK + lane; q < p; q += 64)
-    c += w.tok[q] != INVALID_ID;
+#pragma unroll
+  for (int j = 0; j < STEPS; ++j) {
+    const int q = 4 * (tid + j * COMPACT_TPB);
+    c += (q < n && v[j].x != INVALID_ID) + (q + 1 < n && v[j].y != INVALID_ID) +
+         (q + 2 < n && v[j].z != INVALID_ID) + (q + 3 < n && v[j].w != INVALID_ID);
+  }
   for (int o = 32; o > 0; o >>= 1) c += (uint32_t)__shfl_xor((int)c, o);
-  if (lane == 0) rows[d] = (uint64_t)w.blkprefix[blk] + c;
+  if ((tid & 63) == 0) part[tid >> 6] = c;
+  __syncthreads();
+  if (tid == 0) {
+    for (int k = 1; k < WAVES; ++k) c += part[k];
+    rows[d] = (uint64_t)w.blkprefix[blk] + c;
+  }
 }
 
 // the document-start mask of a batch from its offsets: one thread per mask
@@ -5175,9 +5197,13 @@ hipError_t launch_doc_mask(uint64_t* mask, int64_t nwords,
 hipError_t launch_doc_offsets(const DevWork& w, const uint64_t* doc_offsets,
                               uint32_t n_docs, uint64_t* row_offsets,
                               hipStream_t s) {
-  const uint32_t n = n_docs + 1;  // rows, one wave each
-  hipLaunchKernelGGL(k_doc_offsets, dim3((n + 3) / 4), dim3(256), 0, s, w,
-                     doc_offsets, n_docs, row_offsets);
+  // rows, one workgroup each, in launches of at most 2^22 workgroups (grid size
+  // times workgroup size stays below 2^32)
+  constexpr uint32_t CHUNK = 1u << 22;
+  const uint64_t rows = (uint64_t)n_docs + 1;
+  for (uint64_t at = 0; at < rows; at += CHUNK)
+    hipLaunchKernelGGL(k_doc_offsets, dim3((uint32_t)(rows - at < CHUNK ? rows - at : CHUNK)),
+                       dim3(COMPACT_TPB), 0, s, w, doc_offsets + at, row_offsets + at);
   return hipGetLastError();
 }
 
