@@ -87,7 +87,7 @@ def test_largest_small_tile_request(name, past):
 @pytest.mark.parametrize("name", NAMES)
 def test_whitespace_runs_across_words(name):
     """Whitespace runs with CR/LF that reach one or more 64-byte words past
-    the character asking about them, at every alignment, ended by letters,
+    the character asking about them, at drawn alignments, ended by letters,
     punctuation, non-ASCII characters and whitespace, the text's end, and
     (as documents of one batch) a document's start."""
     rng = np.random.default_rng(72)
@@ -104,3 +104,53 @@ def test_whitespace_runs_across_words(name):
     check(name, "".join(docs), "joined")
     for k, (d, got) in enumerate(zip(docs, tok(name).encode_batch(docs))):
         assert np.array_equal(got.array, kit(name).expected(d)), (name, k)
+
+
+def _start_showing(js: str) -> str:
+    """A variant of an artifact whose only merges join a CR/LF and the blank
+    after it: such a blank starts a piece exactly when its id is its own."""
+    import json
+    from toktier_amd import bpe_tables
+    b2u = bpe_tables.bytes_to_unicode()
+    spec = json.loads(js)
+    merges = [[b2u[a], b2u[b]] for a in b"\n\r" for b in b" \t"]
+    toks = [b2u[b] for b in range(256)] + [a + b for a, b in merges]
+    spec["model"]["vocab"] = {t: i for i, t in enumerate(toks)}
+    spec["model"]["merges"] = merges
+    return json.dumps(spec)
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_crlf_runs_at_every_offset(name):
+    """Blanks right after a CR/LF run at each of the 64 offsets of a word,
+    after every kind of character, in one text (large tiles) and in a request
+    that takes the small tiles."""
+    import itertools
+    import toktier_amd
+    from oracle.oracle import Oracle
+    from toktier_amd import bpe_tables, classes, families
+    js = _start_showing(kit(name).json)
+    f, tables = kit(name).family, bpe_tables.load_tables(js)
+    o = Oracle(tables, classes.table_named(families.class_table_name(f)),
+               classes.nfc_qc_table(), f.ruleset, f.digits_max, f.needs_nfc,
+               contractions=f.contractions)
+    t = toktier_amd.load(name, tokenizer_json=js)
+    o.set_added([a.content.encode() for a in t.added_tokens],
+                [a.id for a in t.added_tokens])
+    docs, at = [], 0
+    for k, unit in enumerate(itertools.product(
+            ["a", "!", "！", " ", "1", ""], ["\n", "\r\n", "\n\r" * 33],
+            [" ", "    ", "\t" + " " * 65], ["\nfoo", "foo", "\r\n!", "é", "　\n"])):
+        body = "".join(unit).encode()
+        before = len((unit[0] + unit[1]).encode())
+        for off in range(64):  # the first blank's offset in its word
+            lead = (off - at - before) % 64 + 64 * (k % 2)
+            docs.append(b"x" * lead + body)
+            at += len(docs[-1])
+    small = docs[::2][:len(docs) * SMALL_MAX // (2 * at)]
+    for part in (docs, small):
+        joined = b"".join(part)
+        assert (len(joined) <= SMALL_MAX) == (part is small)
+        got = t.encode(joined.decode()).array
+        assert np.array_equal(got, o.encode_bytes(joined)), name
+    t.close()

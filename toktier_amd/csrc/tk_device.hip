@@ -1613,14 +1613,16 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
         // staged bytes from HBM, held the whole tile up: 4,194,304 chars of
         // code took 134 us here, 75 with these masks; 20,011 chars 41 -> 17).
         uint64_t nWS = 0, nCR = 0, nHI = 0, pWS = 0, pCR = 0, pHI = 0;
-        if (__builtin_amdgcn_ballot_w64(open && r == FAST_CRLF)) {
+        const uint64_t ask = __builtin_amdgcn_ballot_w64(open && r == FAST_CRLF);
+        if (ask) {
           if ((mWS | mCR) >> 63) {
             const uint32_t b = sb[sj + 64];
             nWS = __ballot(b == ' ' || b == '\t' || b == 0x0B || b == 0x0C);
             nCR = __ballot(b == '\n' || b == '\r');
             nHI = __ballot(b >= 0x80);
           }
-          if (mCR & 1) {
+          // (the CR/LF before the word's first character lies in the word before)
+          if ((mCR | ask) & 1) {
             const uint32_t b = sb[sj - 64];
             pWS = __ballot(b == ' ' || b == '\t' || b == 0x0B || b == 0x0C);
             pCR = __ballot(b == '\n' || b == '\r');
