@@ -123,8 +123,9 @@ def _start_showing(js: str) -> str:
 @pytest.mark.parametrize("name", NAMES)
 def test_crlf_runs_at_every_offset(name):
     """Blanks right after a CR/LF run at each of the 64 offsets of a word,
-    after every kind of character, in one text (large tiles) and in a request
-    that takes the small tiles."""
+    after every kind of character, in one text (large tiles), in a request
+    that takes the small tiles, and as documents of one batch, each of which
+    starts 0 to 127 bytes before its case."""
     import itertools
     import toktier_amd
     from oracle.oracle import Oracle
@@ -153,4 +154,9 @@ def test_crlf_runs_at_every_offset(name):
         assert (len(joined) <= SMALL_MAX) == (part is small)
         got = t.encode(joined.decode()).array
         assert np.array_equal(got, o.encode_bytes(joined)), name
+        ids, rows, status = t.engine.encode_batch(part)
+        assert not status.any()
+        for k, d in enumerate(part):
+            want = o.encode_bytes(d)
+            assert np.array_equal(ids[int(rows[k]):int(rows[k + 1])], want), (name, k, d)
     t.close()

@@ -16,8 +16,9 @@ The model restates the decision with the device's bit arithmetic and checks
 every answer against the oracle's split, for runs at all 64 offsets of a
 word, with and without document starts around them. Planted mistakes must
 each answer some position wrongly: the masks of the word before not read for
-the word's first character, document starts in the word before not read, and
-those in the next word not read.
+the word's first character, a mask shifted by 64 that comes out full instead
+of empty, document starts in the word before not read, and those in the next
+word not read.
 """
 
 from __future__ import annotations
@@ -51,8 +52,10 @@ def doc_word(docs, wd: int) -> int:
     return sum(1 << (d & 63) for d in docs if d >> 6 == wd)
 
 
-def lanes_from(lo: int) -> int:
-    """Bits lo..63; none for lo 64."""
+def lanes_from(lo: int, plant=None) -> int:
+    """Bits lo..63; none for lo 64 (the planted shift wraps around)."""
+    if plant == "shift_by_64":
+        lo &= 63
     return ALL & ~((1 << lo) - 1)
 
 
@@ -104,7 +107,7 @@ def decide(data, docs, i, is_p, plant=None):
             return None
         q = (~pcr & ALL).bit_length() - 1
         dmp = 0 if plant == "docs_before" else doc_word(docs, wd - 1)
-        if dmp & lanes_from(q + 1) or (pws >> q) & 1:
+        if dmp & lanes_from(q + 1, plant) or (pws >> q) & 1:
             return 0
         return None if (phi >> q) & 1 else int(is_p(data[64 * (wd - 1) + q]))
     if fd <= f and fd != 64 and fd < 128:
@@ -206,7 +209,8 @@ def test_hint_matches_a_walk():
     assert known > 10_000
 
 
-@pytest.mark.parametrize("plant", ["first_char", "docs_before", "next_docs"])
+@pytest.mark.parametrize("plant", ["first_char", "shift_by_64", "docs_before",
+                                   "next_docs"])
 def test_planted_mask_mistakes_are_caught(plant):
     o, is_p = kit("qwen3_8b").oracle, ascii_p("qwen3_8b")
     for data, docs in cases():

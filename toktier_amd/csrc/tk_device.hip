@@ -195,7 +195,7 @@ __device__ __forceinline__ uint64_t mask_le(int lane) {
   return lane == 63 ? ~0ULL : ((2ULL << lane) - 1);
 }
 
-__device__ __forceinline__ uint64_t lanes_in(int lo, int hi) {  // [lo, hi)
+__device__ __forceinline__ uint64_t lanes_in(int lo, int hi) {  // [lo, hi), lo < 64
   const uint64_t up = hi >= 64 ? ~0ULL : ((1ULL << hi) - 1);
   return up & ~((1ULL << lo) - 1);
 }
@@ -1676,7 +1676,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
               } else if (~pCR) {
                 const int q = 63 - __builtin_clzll(~pCR);  // in the word before
                 const uint64_t dmp = D ? sdm[wd - 1 - wlo] : 0;
-                if ((dmp & lanes_in(q + 1, 64)) || ((pWS >> q) & 1)) r = 0;
+                if ((dmp & ~mask_le(q)) || ((pWS >> q) & 1)) r = 0;
                 else if (!((pHI >> q) & 1)) r = kcl(se[Li - lane - 64 + q]) == KP;
               }
             } else if (fd <= f && fd != 64 && fd < 128) {
