@@ -25,7 +25,7 @@ def _const(name: str) -> str:
     return re.search(rf"constexpr \w+ {name} =\s*([^;]+);", h.read_text()).group(1)
 
 
-TILE_S = int(_const("PT_TILE_S"))
+TILE, TILE_S = int(_const("PT_TILE")), int(_const("PT_TILE_S"))
 SMALL_MAX = TILE_S * 256 * 7  # PT_SMALL_MAX
 
 _TOKS: dict = {}
@@ -69,6 +69,17 @@ def test_runs_across_many_small_tiles(name):
                 " " * 3000 + "\n" + "\t" * 3000, "\r\n" * 2000, "Q" * n + "é"):
         for lead in ("", "ab ", "!"):
             check(name, lead + run + " z1", (run[:2], lead))
+
+
+@pytest.mark.parametrize("name", NAMES)
+def test_runs_across_large_tiles(name):
+    """Such runs in a request on large tiles, whose o200k / kimi look-back
+    takes a tile a step."""
+    n = 5 * TILE + 37
+    lead = "ab 12 " * (SMALL_MAX // 6 + 1)
+    for run in ("1234567" * (n // 7), "中" * (n // 3), "!́" * (n // 3),
+                " " * 6000 + "\n" + "\t" * 6000, "\r\n" * 4000, "Q" * n + "é"):
+        check(name, lead + run + " z1 " + run + "!", run[:2])
 
 
 @pytest.mark.parametrize("name", NAMES)

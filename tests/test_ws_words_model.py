@@ -115,15 +115,26 @@ def decide(data, docs, i, is_p, plant=None):
     return None if fhi else 1
 
 
-def hint(data, docs, i, plant=None):
+def hint(data, docs, i):
     """The o200k / kimi answer: 0 (another CR/LF follows), 1 (none does) or
     None (walked)."""
-    f, fd, g, fhi = ahead(data, docs, i, plant)
-    if g < min(f, fd):
+    wd, lane = i >> 6, i & 63
+    ws, cr, hi = masks(data, wd)
+    above = ALL & ~((2 << lane) - 1)
+    ns, dm = ~(ws | cr) & ALL, doc_word(docs, wd)
+    low = (ns | dm) & above
+    low &= -low
+    if cr & above & (low - 1):
         return 0
-    if fd <= f and fd != 64 and fd < 128:
+    if low & (dm | ~hi):
         return 1
-    return 1 if f != 64 and not fhi else None
+    if low == 0 and (cr > ns or ns == 0):
+        ws, cr, hi = masks(data, wd + 1)
+        dm = doc_word(docs, wd + 1)
+        end = (~(ws | cr) & ALL) | dm
+        end &= -end
+        return 0 if cr & (end - 1) else 1 if end & (dm | ~hi) else None
+    return None
 
 
 def asking(data, docs):

@@ -1772,7 +1772,7 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
   // tile) and carries the state from word to word. Its entry state is the
   // function of the word before its block when that function is constant
   // (on ordinary text it is). Otherwise every wave first composes its
-  // block's function, and thread 0 takes the tile's entry from the word
+  // block's function, and wave 0 takes the tile's entry from the word
   // before the tile or from the tiles before it (each tile publishes its
   // whole function before it looks back, and the state after it once
   // known: a decoupled look-back with bounded waits) and derives the
@@ -1806,29 +1806,24 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
         const uint64_t mCR = __ballot(bb == '\n' || bb == '\r');
         const uint64_t mHI = __ballot(bb >= 0x80);
         const uint64_t above = ~mask_le(lane);
-        const uint64_t stop = ~(mWS | mCR) & above;
-        int fs = stop ? __builtin_ctzll(stop) : 64;
-        const uint64_t dmw = D ? sdm[(base >> 6) + k - wlo] & above : 0;
-        int fd = dmw ? __builtin_ctzll(dmw) : 64;
-        int gc = (mCR & above) ? __builtin_ctzll(mCR & above) : 64;
-        bool hi = fs < 64 && ((mHI >> fs) & 1);
-        if ((mWS | mCR) >> 63) {  // (wave-uniform) the run goes on in the next word
+        // the run's end: its first byte that is no whitespace, or a document
+        // start (low: that bit, 0 when the run reaches the word's end)
+        const uint64_t ns = ~(mWS | mCR), dm = D ? sdm[(base >> 6) + k - wlo] : 0;
+        const uint64_t first = (ns | dm) & above, low = first & (0 - first);
+        if (mCR & above & (low - 1)) ws_hint = 0;
+        else if (low & (dm | ~mHI)) ws_hint = 1;
+        // (wave-uniform, rare) the word's last run holds a CR/LF, or is the
+        // whole word: the characters of it may ask about the next word
+        if (__builtin_expect(mCR > ns || ns == 0, 0)) {
           const uint32_t b = sb[64 * (k + 1) + lane + PT_PAD];
           const uint64_t nWS = __ballot(b == ' ' || b == '\t' || b == 0x0B || b == 0x0C);
           const uint64_t nCR = __ballot(b == '\n' || b == '\r');
           const uint64_t nHI = __ballot(b >= 0x80);
-          if (fs == 64 && fd == 64 && gc == 64) {
-            const uint64_t ns = ~(nWS | nCR), dmn = D ? sdm[(base >> 6) + k + 1 - wlo] : 0;
-            fs = ns ? 64 + __builtin_ctzll(ns) : 128;
-            fd = dmn ? 64 + __builtin_ctzll(dmn) : 128;
-            gc = nCR ? 64 + __builtin_ctzll(nCR) : 128;
-            hi = ns == 0 || ((nHI >> (fs & 63)) & 1);
-          }
+          const uint64_t dmn = D ? sdm[(base >> 6) + k + 1 - wlo] : 0;
+          const uint64_t end = ~(nWS | nCR) | dmn, nlow = end & (0 - end);
+          const int next = (nCR & (nlow - 1)) ? 0 : (nlow & (dmn | ~nHI)) ? 1 : -1;
+          if (first == 0 && ws_hint < 0) ws_hint = next;
         }
-        const int end = fd < fs ? fd : fs;  // the run's end, as far as the masks go
-        if (gc < end) ws_hint = 0;
-        else if (fd <= fs && fd != 64 && fd < 128) ws_hint = 1;
-        else if (fs != 64 && !hi) ws_hint = 1;
       }
       *f = o2_ident<W>();
       *g = 0;
@@ -1956,62 +1951,115 @@ __global__ __launch_bounds__(PRETOK_TPB) __attribute__((amdgpu_waves_per_eu(7, 7
       if (lane == 0)
         for (int q = 0; q < W; ++q) o2b[wv][q] = B.d[q];
       __syncthreads();
-      if (wv == 0) {
-        Fn A = lds_fn(o2b, 0);
-        for (int j = 1; j < PRETOK_TPB / 64; ++j) A = o2_then(A, lds_fn(o2b, j));
-        uint32_t entry;
-        const Fn H = lds_fn(o2w, 0);
-        if (o2_const<RS>(H)) {
-          entry = o2_at(H, 0);
-        } else {
-          if (lane == 0) o2_publish(op, w.seq, O2_AGG, o2_pack<RS>(A), 0);
-          // G: the function of the tiles looked at, up to this one. 64
-          // tiles a step, lane 63 the nearest (lanes in text order, so the
-          // wave's scan composes them): only the tiles after the last one
-          // whose function is constant have to be published. (One tile a
-          // step waited on its predecessor's in turn, a round trip each.)
-          Fn G = o2_ident<W>();
-          WaitBound wb;
-          bool stall = false;
-          for (int64_t top = (int64_t)blockIdx.x - 1; !o2_const<RS>(G) && !stall;
-               top -= 64) {
-            const int64_t u = top - 63 + lane;
-            // (before tile 0 nothing came: position 0 starts a document)
-            bool pub = u < 0;
-            Fn f = u < 0 ? o2_rep<W>(O2_FRESH) : o2_ident<W>();
-            for (;;) {
-              if (!pub) {
-                const uint64_t* q = w.ostate + 2 * u;
-                const uint64_t v1 =
-                    __hip_atomic_load(q + 1, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
-                pub = (uint32_t)(v1 >> 32) == w.seq;
-                if (pub && ((v1 >> 30) & 3) == O2_INCL) {
-                  f = o2_rep<W>((uint32_t)(v1 >> 26) & 15);
-                } else if (pub) {
-                  const uint64_t v0 =
-                      __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                  f = o2_unpack<RS>((uint32_t)v0 | ((v1 & 0xFFFFF) << 32));
+      // The tile's entry. On large tiles thread 0 looks back a tile a step; a
+      // run spans 3.7 times as many small ones, where a tile a step waited on
+      // its predecessor's in turn, a round trip each, so wave 0 looks at 64.
+      // (That code in the large tiles' kernel costs its every word: with it
+      // 4,194,304 chars of prose took 239 us on gpt_oss and 260 on kimi, 235
+      // and 257 without.)
+      if constexpr (TILE == PT_TILE) {
+        if (tid == 0) {
+          Fn A = lds_fn(o2b, 0);
+          for (int j = 1; j < PRETOK_TPB / 64; ++j) A = o2_then(A, lds_fn(o2b, j));
+          uint32_t entry = O2_FRESH;
+          const Fn H = lds_fn(o2w, 0);
+          if (o2_const<RS>(H)) {
+            entry = o2_at(H, 0);
+          } else {
+            o2_publish(op, w.seq, O2_AGG, o2_pack<RS>(A), 0);
+            // G: the function of the tiles after u up to this one
+            Fn G = o2_ident<W>();
+            bool done = false;
+            WaitBound wb;
+            for (int64_t u = (int64_t)blockIdx.x - 1; u >= 0 && !done; --u) {
+              const uint64_t* q = w.ostate + 2 * u;
+              uint64_t v1;
+              while ((uint32_t)((v1 = __hip_atomic_load(q + 1, __ATOMIC_ACQUIRE,
+                                                        __HIP_MEMORY_SCOPE_AGENT)) >> 32) !=
+                     w.seq) {
+                if (wb.expired(w.wait_ticks)) break;
+                __builtin_amdgcn_s_sleep(2);
+              }
+              if ((uint32_t)(v1 >> 32) != w.seq) {
+                st |= ST_STALL_PRETOK;
+                done = true;
+              } else if (((v1 >> 30) & 3) == O2_INCL) {
+                entry = o2_at(G, (uint32_t)(v1 >> 26) & 15);
+                done = true;
+              } else {
+                const uint64_t v0 = __hip_atomic_load(q, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+                G = o2_then(o2_unpack<RS>((uint32_t)v0 | ((v1 & 0xFFFFF) << 32)), G);
+                if (o2_const<RS>(G)) {
+                  entry = o2_at(G, 0);
+                  done = true;
                 }
               }
-              const uint64_t cm = __ballot(pub && o2_const<RS>(f));
-              const int last = cm ? 63 - __builtin_clzll(cm) : -1;
-              if (!__ballot(!pub && lane > last)) break;
-              if (__any(wb.expired(w.wait_ticks))) {
-                stall = true;
-                break;
-              }
-              __builtin_amdgcn_s_sleep(2);
             }
-            G = o2_then(o2_lane63(o2_scan(f)), G);
+            // (past tile 0 nothing came before: position 0 starts a document)
+            if (!done) entry = o2_at(G, O2_FRESH);
           }
-          if (stall) st |= ST_STALL_PRETOK;
-          entry = o2_at(G, O2_FRESH);
-        }
-        if (lane == 0) {
           o2_publish(op, w.seq, O2_INCL, 0, o2_at(A, entry));
           o2e[0] = entry;
-          for (int j = 1; j < PRETOK_TPB / 64; ++j)
-            o2e[j] = o2_at(lds_fn(o2b, j - 1), o2e[j - 1]);
+          for (int j = 1; j < PRETOK_TPB / 64; ++j) o2e[j] = o2_at(lds_fn(o2b, j - 1), o2e[j - 1]);
+        }
+      } else {
+        if (wv == 0) {
+          Fn A = lds_fn(o2b, 0);
+          for (int j = 1; j < PRETOK_TPB / 64; ++j) A = o2_then(A, lds_fn(o2b, j));
+          uint32_t entry;
+          const Fn H = lds_fn(o2w, 0);
+          if (o2_const<RS>(H)) {
+            entry = o2_at(H, 0);
+          } else {
+            if (lane == 0) o2_publish(op, w.seq, O2_AGG, o2_pack<RS>(A), 0);
+            // G: the function of the tiles looked at, up to this one. 64
+            // tiles a step, lane 63 the nearest (lanes in text order, so the
+            // wave's scan composes them): only the tiles after the last one
+            // whose function is constant have to be published.
+            Fn G = o2_ident<W>();
+            WaitBound wb;
+            bool stall = false;
+            for (int64_t top = (int64_t)blockIdx.x - 1; !o2_const<RS>(G) && !stall;
+                 top -= 64) {
+              const int64_t u = top - 63 + lane;
+              // (before tile 0 nothing came: position 0 starts a document)
+              bool pub = u < 0;
+              Fn f = u < 0 ? o2_rep<W>(O2_FRESH) : o2_ident<W>();
+              for (;;) {
+                if (!pub) {
+                  const uint64_t* q = w.ostate + 2 * u;
+                  const uint64_t v1 =
+                      __hip_atomic_load(q + 1, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+                  pub = (uint32_t)(v1 >> 32) == w.seq;
+                  if (pub && ((v1 >> 30) & 3) == O2_INCL) {
+                    f = o2_rep<W>((uint32_t)(v1 >> 26) & 15);
+                  } else if (pub) {
+                    const uint64_t v0 =
+                        __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    f = o2_unpack<RS>((uint32_t)v0 | ((v1 & 0xFFFFF) << 32));
+                  }
+                }
+                const uint64_t cm = __ballot(pub && o2_const<RS>(f));
+                const int last = cm ? 63 - __builtin_clzll(cm) : -1;
+                if (!__ballot(!pub && lane > last)) break;
+                if (__any(wb.expired(w.wait_ticks))) {
+                  stall = true;
+                  break;
+                }
+                __builtin_amdgcn_s_sleep(2);
+              }
+              G = o2_then(o2_lane63(o2_scan(f)), G);
+            }
+            if (stall) st |= ST_STALL_PRETOK;
+            entry = o2_at(G, O2_FRESH);
+          }
+          if (lane == 0) {
+            o2_publish(op, w.seq, O2_INCL, 0, o2_at(A, entry));
+            o2e[0] = entry;
+            for (int j = 1; j < PRETOK_TPB / 64; ++j)
+              o2e[j] = o2_at(lds_fn(o2b, j - 1), o2e[j - 1]);
+          }
         }
       }
       __syncthreads();
