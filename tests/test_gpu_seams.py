@@ -105,6 +105,24 @@ def test_long_pieces_between_seams(name):
             assert np.array_equal(tok(name).encode(text).array, want), (name, k)
 
 
+@pytest.mark.parametrize("name", ["qwen3_8b", "deepseek_v3", "gpt_oss_120b"])
+def test_split_with_and_without_long_pieces(name):
+    """Split pieces with parts over 128 bytes, in turn without and with a
+    piece over 512: the merges of those parts and the long pieces' chain take
+    the same side stream."""
+    rng = np.random.default_rng(34)
+    base = [_letters(name, rng, 512) for _ in range(150)] + ["Qz" * 70, "ab" * 120]
+    for turn in range(6):
+        parts = [base[int(rng.integers(0, len(base)))].encode()[:int(rng.integers(66, 512))]
+                 .decode("utf-8", "ignore") for _ in range(ROWS_MAX + 40)]
+        if turn % 2:
+            parts[turn * 100] = _letters(name, rng, 3000)
+        text = "\n".join(parts)
+        want = kit(name).expected(text)
+        assert not isinstance(want, int)
+        assert np.array_equal(tok(name).encode(text).array, want), (name, turn)
+
+
 def test_dropped_bytes_and_boundary_table_take_no_parts():
     """An artifact that drops bytes and the boundary-format pair table keep
     the general merges, on text that the split would take."""

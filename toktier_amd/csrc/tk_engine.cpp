@@ -435,6 +435,7 @@ struct tk_engine {
   // their own, beside the 129..WIDE_MAX-byte merges of stream2
   hipStream_t stream3 = nullptr;
   hipEvent_t ev_join3 = nullptr;
+  hipEvent_t ev_split = nullptr;  // the pieces are split (stream2 -> stream3)
   // host-to-host entries: pinned staging of the request bytes and of the
   // ids (written there by the compaction kernel), and the copy threads
   tk::PinnedBuf pin_in, pin_out;
@@ -765,12 +766,26 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
     // the merges of the queued pieces next (after the chain's first kernel,
     // so that one is dispatched first; their launches are not held behind
     // the chain's twenty-odd launches on the host)
+    // The parts over 128 bytes need the split alone: with no chain on its
+    // stream they are merged there, beside the shorter parts. (Behind them,
+    // CJK text of 850,000 to 1,150,000 chars took longer than whole pieces
+    // merged by rows: on DeepSeek 358 / 397 / 432 us by rows, 457 / 456 / 455
+    // split with the rows last, 354 / 365 / 365 with the rows beside.)
+    hipStream_t sr = split && rows && !big ? s3 : s2;
     if (split) HIP_TRY(tk::launch_piece_split(e->t, w, s2, nlong));
+    if (sr != s2) {
+      HIP_TRY(hipEventRecord(e->ev_split, s2));
+      HIP_TRY(hipStreamWaitEvent(sr, e->ev_split, 0));
+    }
     if (split || nmid) HIP_TRY(tk::launch_bpe_mid(e->t, w, s2, split, nmid));
     if (rows) {
-      HIP_TRY(tk::launch_bpe_rows(e->t, w, s2, nlong, split, ks(TK_KERNEL_BPE_ROWS),
+      HIP_TRY(tk::launch_bpe_rows(e->t, w, sr, nlong, split, ks(TK_KERNEL_BPE_ROWS),
                                   ke(TK_KERNEL_BPE_ROWS)));
       launched[TK_KERNEL_BPE_ROWS] = true;
+    }
+    if (sr != s2) {
+      HIP_TRY(hipEventRecord(e->ev_join3, sr));
+      HIP_TRY(hipStreamWaitEvent(s, e->ev_join3, 0));
     }
     if (big) {
       HIP_TRY(tk::launch_long_segments(e->t, w, s3));
@@ -1175,6 +1190,8 @@ int tk_engine_open(const tk_config* cfg, const uint8_t* class_table,
   if (hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming |
                                                hipEventDisableSystemFence) != hipSuccess ||
       hipEventCreateWithFlags(&e->ev_join3, hipEventDisableTiming |
+                                                hipEventDisableSystemFence) != hipSuccess ||
+      hipEventCreateWithFlags(&e->ev_split, hipEventDisableTiming |
                                                 hipEventDisableSystemFence) != hipSuccess)
     return bail(fail(TK_E_DEVICE, "hipEventCreateWithFlags failed"));
   for (auto& ev : e->ev)
@@ -1350,6 +1367,7 @@ void tk_engine_close(tk_engine* e) {
   if (e->stream3) (void)hipStreamSynchronize(e->stream3);
   if (e->ev_join) (void)hipEventDestroy(e->ev_join);
   if (e->ev_join3) (void)hipEventDestroy(e->ev_join3);
+  if (e->ev_split) (void)hipEventDestroy(e->ev_split);
   if (e->stream) (void)hipStreamDestroy(e->stream);
   if (e->stream2) (void)hipStreamDestroy(e->stream2);
   if (e->stream3) (void)hipStreamDestroy(e->stream3);
