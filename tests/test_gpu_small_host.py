@@ -1,8 +1,8 @@
 """A small host request's bytes are read by the literal kernel from the pinned
-staging, and its call ends with the outcome words: sizes at the edges of the
-16-byte loads, of the kernel's blocks and of the largest such request, from
-aligned, misaligned and page-locked sources, each buffer refilled between
-calls; against the oracle."""
+staging: sizes at the edges of the 16-byte loads, of the kernel's blocks and
+of the largest such request, from aligned, misaligned and page-locked sources,
+each buffer refilled between calls; and the ids of a call are all there when
+it returns; against the oracle."""
 
 from __future__ import annotations
 
@@ -68,8 +68,8 @@ def test_sizes_and_sources(qwen, n):
 
 
 def test_device_calls_on_two_streams_in_turn(qwen):
-    """A call that ends with its outcome words leaves nothing another stream's
-    next call on the same engine could meet; the ids are read on a third."""
+    """A call leaves nothing another stream's next call on the same engine could
+    meet; the ids are read on a third."""
     import torch
     k, t, base = qwen
     E = t.engine
@@ -86,3 +86,26 @@ def test_device_calls_on_two_streams_in_turn(qwen):
         assert st == 0, (i, E._L.tk_last_error())
         got = ids[i & 1][:m.value].cpu().numpy().view(np.uint32)
         assert np.array_equal(got, k.oracle.encode_bytes(b)), i
+
+
+@pytest.mark.parametrize("locked", [False, True])
+def test_every_id_is_there_when_a_call_returns(qwen, locked):
+    """Small calls in turn whose ids end in a partly filled line of the buffer
+    that the device writes, each other than the one before at that place: an id
+    still on its way when the call returns would show the earlier call's."""
+    import torch
+    k, t, base = qwen
+    E = t.engine
+    texts = [_cut(base, 700 + 37 * i, 977 * i) for i in range(24)]
+    want = [k.oracle.encode_bytes(b) for b in texts]
+    room = max(len(b) for b in texts)
+    out = (torch.zeros(room, dtype=torch.int32, pin_memory=True).numpy().view(np.uint32)
+           if locked else np.zeros(room, dtype=np.uint32))
+    m = C.c_size_t()
+    for i in range(40 * len(texts)):
+        j = 7 * i % len(texts)
+        b, w = texts[j], want[j]
+        st = E._L.tk_engine_encode(E._h, b, len(b), 0, C.c_void_p(out.ctypes.data),
+                                   out.size, C.byref(m))
+        assert st == 0 and m.value == w.size, (i, E._L.tk_last_error())
+        assert np.array_equal(out[:w.size], w), i

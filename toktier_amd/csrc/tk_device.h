@@ -209,8 +209,6 @@ struct DevWork {
                          // line each (ctrl)
   uint32_t* prepdone;    // k_bpe_pack waves done with the long pieces (ctrl)
   uint32_t* gate;        // GATE_WORDS in host memory, or nullptr
-  uint32_t* ndone;       // k_compact's finished blocks (ctrl), when the host
-                         // waits for GATE_DONE alone; nullptr: the stream's end
   uint32_t seq;          // call number written to gate[GATE_SEQ]
   // bound of every wait on another workgroup's published word, in ticks
   // of the device's constant-rate real-time counter (wall_clock64)
@@ -249,7 +247,7 @@ constexpr uint64_t HR_FIRST = 1ull << 31, HR_LAST = 1ull << 30;
 constexpr int CTRL_STATUS = 0, CTRL_TOTAL = 1, CTRL_LONG = 2, CTRL_SEG = 3,
               CTRL_FAIL = 4, CTRL_BIG = 5, CTRL_NLIT = 6, CTRL_PASS = 7,
               CTRL_FAIL2 = 8, CTRL_PREP = 9, CTRL_WIDE = 10, CTRL_ROWS = 11,
-              CTRL_WIN = 12, CTRL_DONE = 13, CTRL_ROWQ = 16,  // (ROWQ: PACK_XCDS words)
+              CTRL_WIN = 12, CTRL_ROWQ = 16,  // (ROWQ: PACK_XCDS words)
               CTRL_VLIST = 24,
               CTRL_PSEG = 64, CTRL_PSEG_STRIDE = 64,
               CTRL_PSEG_COUNT = 32, CTRL_PART = CTRL_PSEG + 8 * CTRL_PSEG_STRIDE,
@@ -407,12 +405,6 @@ __host__ __device__ inline uint32_t pack_seg_list(uint32_t ntile, int x,
 constexpr int COMPACT_TPB = 256;
 constexpr int COMPACT_PER_THREAD = 32;
 constexpr int COMPACT_BLOCK = COMPACT_TPB * COMPACT_PER_THREAD;  // 8192
-// Up to this many compaction blocks the host waits for the outcome words alone
-// (each block counts itself done behind a system-scope fence) and not for the
-// stream's end. The counts are taken one after another at the memory side,
-// ~40 ns each: 16 KiB on the device 75.6 -> 71.3 us and 512 KiB 79.3 -> 78.0,
-// but 1 MiB (128 blocks) 88.2 -> 91.7.
-constexpr int64_t DONE_BLOCKS = 64;
 
 // start / stop: optional timing events taken from the start of the stage's
 // first dispatch / the end of its last one

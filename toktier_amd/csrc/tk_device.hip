@@ -5007,26 +5007,21 @@ __global__ __launch_bounds__(COMPACT_TPB) void k_compact(DevWork w, int64_t nblk
     w.blkprefix[nblk] = total;
     w.status[1] = total;
     if (total > w.out_cap) atomicOr(w.status, ST_CAPACITY);
-  }
-  bool last = b == nblk - 1 && tid == 0;
-  if (w.ndone) {
-    // every block's ids (and the last block's words above) are visible to
-    // the host and the device before it counts itself done
-    __threadfence_system();
-    __syncthreads();
-    last = tid == 0 && atomicAdd(w.ndone, 1u) == (uint32_t)nblk - 1;
-  }
-  if (last && w.gate) {
-    // every earlier stage that sets status bits or failed cuts has ended
-    w.gate[GATE_STATUS] = atomicOr(w.status, 0u);
-    w.gate[GATE_TOTAL] = __hip_atomic_load(w.status + 1, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-    w.gate[GATE_FAIL] = *w.nfail;
-    w.gate[GATE_NLIT] = w.nlit ? *w.nlit : 0u;
-    w.gate[GATE_PASS] = w.npass ? *w.npass : 0u;
-    __threadfence_system();
-    w.gate[GATE_DONE] = w.seq;
-    __threadfence_system();
+    if (w.gate) {
+      // every earlier stage that sets status bits or failed cuts has ended.
+      // The host reads these words after the stream's end, not before: a
+      // call that waited for GATE_DONE alone once read the last ids of its
+      // page-locked buffer before they had arrived there, though every
+      // block's system-scope fence came before the word.
+      w.gate[GATE_STATUS] = atomicOr(w.status, 0u);
+      w.gate[GATE_TOTAL] = total;
+      w.gate[GATE_FAIL] = *w.nfail;
+      w.gate[GATE_NLIT] = w.nlit ? *w.nlit : 0u;
+      w.gate[GATE_PASS] = w.npass ? *w.npass : 0u;
+      __threadfence_system();
+      w.gate[GATE_DONE] = w.seq;
+      __threadfence_system();
+    }
   }
 }
 

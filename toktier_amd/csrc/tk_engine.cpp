@@ -629,28 +629,23 @@ int read_ctrl_words(const uint32_t* ctrl, hipStream_t s, uint32_t* h) {
   return TK_OK;
 }
 
-// Spin on a gate word until the device has written call `seq` there; false
-// after a generous bound (a device fault would stop the writer: the caller
-// then synchronizes the stream, which surfaces its error).
-bool wait_word(tk_engine* e, int word, uint32_t seq) {
+// Wait until k_bpe_pack of call `seq` has written the gate words (a
+// spin on host memory). A device fault would stop the writer, so after a
+// generous bound the stream is synchronized to surface its error.
+int wait_gate(tk_engine* e, uint32_t seq, hipStream_t s) {
   const auto t0 = std::chrono::steady_clock::now();
   for (uint64_t spin = 0;; ++spin) {
-    if (e->gate[word] == seq) {
+    if (e->gate[tk::GATE_SEQ] == seq) {
       std::atomic_thread_fence(std::memory_order_acquire);
-      return true;
+      return TK_OK;
     }
     if ((spin & 1023) == 1023 &&
-        std::chrono::steady_clock::now() - t0 > std::chrono::seconds(10))
-      return false;
+        std::chrono::steady_clock::now() - t0 > std::chrono::seconds(10)) {
+      HIP_TRY(hipStreamSynchronize(s));
+      if (e->gate[tk::GATE_SEQ] == seq) return TK_OK;
+      return fail(TK_E_INTERNAL, "gate words were not written");
+    }
   }
-}
-
-// Wait until k_bpe_pack of call `seq` has written the gate words.
-int wait_gate(tk_engine* e, uint32_t seq, hipStream_t s) {
-  if (wait_word(e, tk::GATE_SEQ, seq)) return TK_OK;
-  HIP_TRY(hipStreamSynchronize(s));
-  if (e->gate[tk::GATE_SEQ] == seq) return TK_OK;
-  return fail(TK_E_INTERNAL, "gate words were not written");
 }
 
 float elapsed_us(hipEvent_t a, hipEvent_t b) {
@@ -816,22 +811,14 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   // the compaction reports the failed cuts left after the last queued pass
   tk::DevWork wc = w;
   if (big) wc.nfail = fail_count(ctrl, DEV_REPAIRS);
-  // a small request with nothing behind its compaction: the outcome words end
-  // the call, 3..4 us before the stream counts as done. Not one whose text was
-  // sent by a copy command: the next call's command then waits for this
-  // kernel's end in the queue (a 64 KiB host call 86 -> 90 us)
-  const bool spin = !rows_out && e->timing == 0 && (src || d_text != ws.text) &&
-                    nb <= (size_t)(tk::DONE_BLOCKS * tk::COMPACT_BLOCK);
-  if (spin) wc.ndone = ctrl + tk::CTRL_DONE;
   HIP_TRY(tk::launch_compact(wc, s, ++ws.ctag, ks(TK_KERNEL_COMPACT),
                              ke(TK_KERNEL_COMPACT)));
   launched[TK_KERNEL_COMPACT] = true;
   if (rows_out)
     HIP_TRY(tk::launch_doc_offsets(w, rows_out->offs, rows_out->n, rows_out->rows, s));
-  wc.ndone = nullptr;
   // k_compact's last block has left the outcome in the gate words: no
   // read-back copy
-  if (!spin || !wait_word(e, tk::GATE_DONE, w.seq)) HIP_TRY(hipStreamSynchronize(s));
+  HIP_TRY(hipStreamSynchronize(s));
   uint32_t* h = e->host_ctrl;
   if (e->gate[tk::GATE_DONE] != w.seq)
     return fail(TK_E_INTERNAL, "outcome words were not written");
@@ -963,8 +950,8 @@ void host_copy(tk_engine* e, uint8_t* dst, const uint8_t* src, size_t n) {
 
 // n request bytes at src (host) into d_dst (device) on stream s: page-locked
 // bytes in one transfer; pageable ones copied into the pinned staging
-// first, then one transfer (the staging is free again once the call's
-// kernels are done with it, which every host entry waits for).
+// first, then one transfer (the staging is free again once the call has
+// synchronized, as every host entry does before it returns).
 int stage_in(tk_engine* e, uint8_t* d_dst, const uint8_t* src, size_t n,
              hipStream_t s) {
   if (pinned_range(src, n)) {
