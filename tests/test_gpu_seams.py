@@ -19,6 +19,7 @@ HEADER = (Path(__file__).resolve().parents[1] / "toktier_amd" / "csrc" /
           "tk_device.h").read_text()
 ROWS_MAX = int(re.search(r"PACK_ROWS_MAX = (\d+);", HEADER).group(1))
 MID_MAX = int(re.search(r"PACK_MID_MAX = (\d+);", HEADER).group(1))
+MID_MAX_SPLIT = int(re.search(r"PACK_MID_MAX_SPLIT = (\d+);", HEADER).group(1))
 
 _TOKS: dict = {}
 
@@ -79,6 +80,24 @@ def test_listed_pieces_one_a_lane(name, count):
         s = base[int(rng.integers(0, len(base)))]
         s = s.encode()[:int(rng.integers(33, 65))].decode("utf-8", "ignore")
         parts.append(s + "x" * max(0, 33 - len(s.encode())))
+    text = "\n".join(parts)
+    want = kit(name).expected(text)
+    assert not isinstance(want, int)
+    assert np.array_equal(tok(name).encode(text).array, want)
+
+
+@pytest.mark.parametrize("name", ["qwen3_8b", "gpt_oss_120b"])
+@pytest.mark.parametrize("count", [MID_MAX_SPLIT, MID_MAX_SPLIT + 1])
+def test_listed_pieces_beside_split_ones(name, count):
+    """The same where longer pieces are split, at the count for that."""
+    rng = np.random.default_rng(35)
+    base = [_letters(name, rng, 130) for _ in range(300)]
+    cut = lambda lo, hi: base[int(rng.integers(0, len(base)))].encode()[  # noqa: E731
+        :int(rng.integers(lo, hi))].decode("utf-8", "ignore")
+    parts = [cut(70, 131) for _ in range(ROWS_MAX + 40)]
+    mid = [cut(36, 65) for _ in range(count)]
+    for k, s in enumerate(mid):
+        parts.insert(2 * k, s + "x" * max(0, 33 - len(s.encode())))
     text = "\n".join(parts)
     want = kit(name).expected(text)
     assert not isinstance(want, int)

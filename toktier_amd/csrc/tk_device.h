@@ -300,9 +300,20 @@ constexpr int PACK_BLOCKS = 1792;
 // k_bpe_mid do (k_bpe_rows, for tables that those do not take)
 constexpr int PACK_ROWS_MAX = 8192;
 // k_bpe_pack merges the pieces of 33..64 bytes (class PACK_MID), one a wave,
-// when there are at most this many; else k_bpe_mid does, one a lane
-constexpr int PACK_MID_MAX = 4096;
+// when there are at most pack_mid_max of them (nlong: the queued pieces over 64
+// bytes); else k_bpe_mid does, one a lane: up to 63 merges in turn, ~60 us
+// however many there are, behind the gate. 5,200 / 8,750 / 10,800 / 13,500
+// words of 33-64 letters: 81 / 96 / 104 / ~117 us by waves, 124 / 125 / 123 /
+// 127 by lanes; 10,700 equal 60-character rules, 135 and 124. With more than
+// PACK_ROWS_MAX queued pieces k_bpe_mid runs in any case: CJK text of
+// 1,400,000 / 2,000,000 chars (4,800 / 6,800 such pieces) 360 / 398 us by
+// lanes, 373 / 419 by waves.
+constexpr int PACK_MID_MAX = 12288;
+constexpr int PACK_MID_MAX_SPLIT = 4096;
 constexpr int PACK_MID = PACK_CLASSES - 1;
+__host__ __device__ __forceinline__ uint32_t pack_mid_max(uint32_t nlong) {
+  return nlong > (uint32_t)PACK_ROWS_MAX ? PACK_MID_MAX_SPLIT : PACK_MID_MAX;
+}
 // The piece lists come in PACK_XCDS segments: segment x holds the pieces of
 // the k_pretok tiles b with b % PACK_XCDS == x (those of one XCD: workgroups
 // go to the XCDs in turn), and the k_bpe_pack blocks of the same residue

@@ -2787,12 +2787,12 @@ void k_bpe_pack(DevTables t, DevWork w) {
   if (nl > w.long_cap) nl = w.long_cap;
   if (wv == 0) {
     uint32_t cnt = cl ? seg[CTRL_PSEG_COUNT + lane] : 0u;
-    // (more than PACK_MID_MAX pieces of 33..64 bytes go to k_bpe_mid)
+    // (more than pack_mid_max pieces of 33..64 bytes go to k_bpe_mid)
     const uint32_t mid = wave_incl_scan(
         lane < PACK_XCDS ? w.pseg[lane * CTRL_PSEG_STRIDE + CTRL_PSEG_COUNT + PACK_MID] : 0u,
         lane);
     if (lane == PACK_MID && mid_table(t) &&
-        __builtin_amdgcn_readlane((int)mid, PACK_XCDS - 1) > PACK_MID_MAX)
+        (uint32_t)__builtin_amdgcn_readlane((int)mid, PACK_XCDS - 1) > pack_mid_max(nl))
       cnt = 0;
     const uint32_t geo = cl ? PACK_GEO[lane] : 0u;
     const uint32_t per = cl ? (geo >> 8) & 0xFF : 1u;

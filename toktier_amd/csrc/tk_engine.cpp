@@ -736,12 +736,13 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   e->last_nlong = nlong;
   e->last_big = e->gate[tk::GATE_BIG];
   // (past PACK_ROWS_MAX the queued pieces are cut at their seams and merged
-  // part by part, or whole by k_bpe_rows; past PACK_MID_MAX the listed ones
+  // part by part, or whole by k_bpe_rows; past pack_mid_max the listed ones
   // of 33..64 bytes are k_bpe_mid's)
   const bool many = nlong > (uint32_t)tk::PACK_ROWS_MAX;
   const bool split = many && tk::mid_table(e->t);
-  const uint32_t nmid = tk::mid_table(e->t) && e->gate[tk::GATE_NMID] > (uint32_t)tk::PACK_MID_MAX
-                            ? e->gate[tk::GATE_NMID] : 0;
+  const uint32_t listed = e->gate[tk::GATE_NMID];
+  const uint32_t nmid =
+      tk::mid_table(e->t) && listed > tk::pack_mid_max(nlong) ? listed : 0;
   // (a part over 128 bytes is of a piece over 128 bytes)
   const bool rows = nrows > 0 || (split ? nwide > 0 : many);
   const bool side2 = split || nmid || rows || nwide > 0 ||
