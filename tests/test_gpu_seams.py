@@ -142,6 +142,41 @@ def test_split_with_and_without_long_pieces(name):
         assert np.array_equal(tok(name).encode(text).array, want), (name, turn)
 
 
+def test_pieces_of_a_table_without_seams(monkeypatch):
+    """Rules with an id of two spellings get no seam tables: the pieces that
+    would be split go uncut, as one part each, to the same kernels."""
+    import dataclasses
+    import toktier_amd
+    from oracle.oracle import Oracle
+    from toktier_amd import bpe_tables, classes, families
+    k = kit("qwen3_8b")
+    t, f = k.tables, k.family
+    used = t.pair_keys[t.pair_keys != 2**64 - 1]
+    sides = np.concatenate([used >> np.uint64(32), used & np.uint64(0xFFFFFFFF)])
+    prod = t.pair_vals & np.uint64(0xFFFFFFFF)
+    # two rules whose products nothing consumes: the first takes the second's
+    # product (the ranks' order stays monotone)
+    end = np.flatnonzero((t.pair_keys != 2**64 - 1) & ~np.isin(prod, sides))
+    end = end[np.argsort(t.pair_vals[end])]
+    vals = t.pair_vals.copy()
+    vals[end[0]] = (vals[end[0]] >> np.uint64(32) << np.uint64(32)) | prod[end[1]]
+    other = dataclasses.replace(t, pair_vals=vals)
+    monkeypatch.setattr(bpe_tables, "load_tables", lambda js: other)
+    d = toktier_amd.load("qwen3_8b")
+    o = Oracle(other, classes.table_named(families.class_table_name(f)),
+               classes.nfc_qc_table(), f.ruleset, f.digits_max, f.needs_nfc)
+    rng = np.random.default_rng(36)
+    base = [_letters("qwen3_8b", rng, 512) for _ in range(150)]
+    for hi in (129, 513):  # (the parts over 128 bytes on their own)
+        text = "\n".join(base[int(rng.integers(0, len(base)))].encode()[
+            :int(rng.integers(68, hi))].decode("utf-8", "ignore")
+            for _ in range(ROWS_MAX + 40))
+        want = o.encode_bytes(text.encode())
+        assert not isinstance(want, int)
+        assert np.array_equal(d.encode(text).array, want), hi
+    d.close()
+
+
 def test_dropped_bytes_and_boundary_table_take_no_parts():
     """An artifact that drops bytes and the boundary-format pair table keep
     the general merges, on text that the split would take."""
