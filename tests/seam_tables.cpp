@@ -6,10 +6,10 @@
 extern "C" int seam_tables(const uint64_t* keys, const uint64_t* vals, uint64_t count,
                            const int32_t* byte_id, uint16_t* mask, uint32_t* bits,
                            uint64_t* words) {
-  std::vector<std::string> strings;
-  if (!tk::symbol_strings(keys, vals, count, byte_id, strings)) return 0;
+  tk::Spelled sp;
+  if (!tk::symbol_strings(keys, vals, count, byte_id, sp)) return 0;
   tk::SeamTables t;
-  tk::build_seams(strings, t);
+  tk::build_seams(sp, {}, t);
   std::copy(t.mask.begin(), t.mask.end(), mask);
   std::copy(t.bits.begin(), t.bits.end(), bits);
   *words = t.bits.size();

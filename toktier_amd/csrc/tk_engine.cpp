@@ -1234,17 +1234,21 @@ int tk_engine_open(const tk_config* cfg, const uint8_t* class_table,
   }
   e->t.seam_mask = nullptr;
   {
-    std::vector<std::string> strings;
-    bool plain = tk::symbol_strings(pair_keys, pair_vals, n_pairs, byte_id, strings);
+    // (only the strings' inner positions count, so a vocabulary entry that
+    // its own id's symbol spells adds nothing)
+    tk::Spelled sp;
+    std::vector<std::pair<const uint8_t*, size_t>> more;
+    bool plain = tk::symbol_strings(pair_keys, pair_vals, n_pairs, byte_id, sp);
     for (uint64_t i = 0; plain && cfg->ignore_merges && i < cfg->vocab_count; ++i) {
       if (vocab_keys[i] == ~0ULL) continue;
       const uint64_t off = vocab_vals[i] >> 30, len = (vocab_vals[i] >> 20) & 0x3FF;
       plain = off <= vocab_blob_len && len <= vocab_blob_len - off;
-      if (plain) strings.emplace_back(reinterpret_cast<const char*>(vocab_blob) + off, len);
+      if (plain && len > 1 && !sp.is(vocab_vals[i] & 0xFFFFF, vocab_blob + off, len))
+        more.emplace_back(vocab_blob + off, len);
     }
     if (plain) {
       tk::SeamTables st;
-      tk::build_seams(strings, st);
+      tk::build_seams(sp, more, st);
       if ((rc = up(e->seam_mask, st.mask.data(), st.mask.size())) != TK_OK) return bail(rc);
       if ((rc = up(e->seam_bits, st.bits.data(), st.bits.size())) != TK_OK) return bail(rc);
       e->t.seam_mask = e->seam_mask.p;
