@@ -300,7 +300,10 @@ const char* tk_engine_architecture(const tk_engine* engine); /* "gfx950" */
 #define TK_KERNEL_PRETOK 0       /* k_pretok: pretokenize, list the pieces */
 #define TK_KERNEL_BPE_PACK 1     /* k_bpe_pack: pieces of up to 128 bytes */
 #define TK_KERNEL_COMPACT 2      /* k_compact: ids compacted */
-#define TK_KERNEL_BPE_ROWS 3     /* k_bpe_rows: pieces of 129-256 bytes */
+#define TK_KERNEL_BPE_ROWS 3     /* k_bpe_rows: pieces of 129-256 bytes, or
+                                  * the parts of that length of split ones
+                                  * (whose shorter parts k_piece_split and
+                                  * k_bpe_mid take, timed in [2] only) */
 #define TK_KERNEL_LONG_WINDOWS 4 /* k_long_windows: cuts of pieces > 512 B */
 #define TK_KERNEL_ADDED 5        /* k_added: added-token literal split */
 #define TK_KERNELS 6

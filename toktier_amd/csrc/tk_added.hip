@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void k_added(DevAdded a, DevWork w,
   const int64_t s0 = B - AD_BACK, nb = w.nb;
   // A small host request's bytes are read from the pinned staging and brought
   // to w.text here: no copy command, and no wait between it and this kernel
-  // (64 KiB host to host 86 -> 77 us).
+  // (64 KiB host to host 86 -> 79 us).
   const uint8_t* const src = w.src ? w.src : w.text;
   int hit = 0;
   // (the staging's 16-byte loads all issued before any is used)

@@ -253,10 +253,11 @@ constexpr int CTRL_STATUS = 0, CTRL_TOTAL = 1, CTRL_LONG = 2, CTRL_SEG = 3,
               CTRL_PSEG_COUNT = 32, CTRL_PART = CTRL_PSEG + 8 * CTRL_PSEG_STRIDE,
               CTRL_PART_STRIDE = 32, CTRL_WORDS = CTRL_PART + 7 * CTRL_PART_STRIDE;
 // gate words in host memory: k_bpe_pack writes GATE_NLONG / GATE_NROWS /
-// GATE_NWIDE / GATE_BIG / GATE_NMID and then GATE_SEQ (the host learns, while the packed merge runs,
-// whether the side streams' long-piece stages have any work), k_compact's
-// last block writes the request's outcome (status, id count, failed cuts)
-// and then GATE_DONE, so no copy is needed to read it
+// GATE_NWIDE / GATE_BIG / GATE_NMID and then GATE_SEQ (the host learns, while
+// the packed merge runs, whether the side streams' long-piece stages have any
+// work), k_compact's last block writes the request's outcome (status, id
+// count, failed cuts) and then GATE_DONE, so no copy is needed to read it
+// after the stream's end
 constexpr int GATE_SEQ = 0, GATE_BIG = 1, GATE_STATUS = 2, GATE_TOTAL = 3,
               GATE_FAIL = 4, GATE_DONE = 5, GATE_NLONG = 6, GATE_NLIT = 7,
               GATE_PASS = 8, GATE_NWIDE = 9, GATE_NROWS = 10, GATE_NMID = 11,
@@ -297,7 +298,7 @@ __host__ __device__ __forceinline__ uint32_t added_slot(uint32_t key,
 constexpr int PACK_BLOCKS = 1792;
 // k_bpe_pack merges the queued pieces of 65..128 bytes itself when at most
 // this many pieces over 64 bytes are queued; else k_piece_split and
-// k_bpe_mid do (k_bpe_rows, for tables that those do not take)
+// k_bpe_mid do (k_bpe_rows, for tables that mid_table refuses)
 constexpr int PACK_ROWS_MAX = 8192;
 // k_bpe_pack merges the pieces of 33..64 bytes (class PACK_MID), one a wave,
 // when there are at most pack_mid_max of them (nlong: the queued pieces over 64

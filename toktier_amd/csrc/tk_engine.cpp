@@ -660,9 +660,12 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
   const uint32_t big = cut ? e->gate[tk::GATE_BIG] : 0;
   e->last_nlong = nlong;
   e->last_big = e->gate[tk::GATE_BIG];
-  // (past PACK_ROWS_MAX the queued pieces are cut at their seams and merged
-  // part by part, or whole by k_bpe_rows; past pack_mid_max the listed ones
-  // of 33..64 bytes are k_bpe_mid's)
+  // (past PACK_ROWS_MAX the queued pieces are cut at their seams, or left
+  // whole by a table without any, and merged part by part; by k_bpe_rows for
+  // tables that k_bpe_mid does not take. Past pack_mid_max the listed ones of
+  // 33..64 bytes are k_bpe_mid's. Pieces without a seam inside are the faster
+  // so too: 900,000 bytes of 70-space indentation 535 us by rows, 172 so, of
+  // 80-letter sequences 234 and 177)
   const bool many = nlong > (uint32_t)tk::PACK_ROWS_MAX;
   const bool split = many && tk::mid_table(e->t);
   const uint32_t listed = e->gate[tk::GATE_NMID];
@@ -815,7 +818,7 @@ int run_pipeline(tk_engine* e, Workspace& ws, const uint8_t* d_text,
 // ---- host <-> device through the pinned staging
 constexpr size_t STAGE_SMALL = (size_t)256 << 10;  // one copy, this thread
 // Up to here k_added reads a host call's bytes from the pinned staging: 64 KiB
-// of ascii 86 -> 77 us, 400,000 bytes 108 -> 101, 512 KiB 115 -> 111; 1 MiB
+// of mixed text 86 -> 79 us, 256 KiB 103 -> 98, 512 KiB 122 -> 119; 1 MiB
 // 147 -> 170 (each block reads its margins over PCIe again, and the bytes
 // come only as fast as the blocks in flight ask for them).
 constexpr size_t MAP_SMALL = (size_t)512 << 10;
