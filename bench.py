@@ -128,9 +128,10 @@ def measured_traffic(config: int, kernel: str):
             m = json.load(f)
     except (OSError, ValueError):
         return None
-    if d.get("build_key") != m.get("build_key") or d.get("kernel") != kernel:
+    k = d.get("kernels", {}).get(kernel)
+    if d.get("build_key") != m.get("build_key") or k is None:
         return None
-    return int(d["fetch_bytes"] + d["write_bytes"])
+    return int(k["fetch_bytes"] + k["write_bytes"])
 
 
 # ------------------------------------------------------------ requests
